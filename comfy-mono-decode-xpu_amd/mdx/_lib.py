@@ -165,12 +165,12 @@ def call(name, *args):
 
 
 SRC_Q8, SRC_HR, SRC_XP, SRC_GN = 0, 1, 2, 3
-SRC_INT_ONLY, SRC_TBL, SRC_TBL8, SRC_GDN = 4, 8, 16, 32
+SRC_INT_ONLY, SRC_TBL, SRC_TBL8, SRC_GDN, SRC_B8 = 4, 8, 16, 32, 64
 
 
 def gemv_trace():
     """The GEMV kernel variants this thread launched since the previous call (mdx_gemv_trace): a list of
-    dicts {mfma, src (SRC_Q8 / SRC_HR / SRC_XP), decode ("integral", "table16", "table8" or "generic"),
+    dicts {mfma, src (SRC_Q8 / SRC_HR / SRC_XP), decode ("integral", "table16", "table8", "bytes" or "generic"),
     s_dtype, rows, tpw, ks, red_alias, gdn (a Gated-DeltaNet projection: conv epilogue, gate work-groups)}."""
     buf = (c_int32 * (7 * 64))()
     n = lib().mdx_gemv_trace(buf, 64)
@@ -178,7 +178,7 @@ def gemv_trace():
     for i in range(min(n, 64)):
         mfma, src, sdt, rows, tpw, ks, alias = buf[7 * i:7 * i + 7]
         dec = ("integral" if src & SRC_INT_ONLY else "table16" if src & SRC_TBL else "table8" if src & SRC_TBL8
-               else "generic")
+               else "bytes" if src & SRC_B8 else "generic")
         out.append(dict(mfma=bool(mfma), src=src & 3, decode=dec, s_dtype=sdt, rows=rows, tpw=tpw, ks=ks,
                         red_alias=bool(alias), gdn=bool(src & SRC_GDN)))
     return out
