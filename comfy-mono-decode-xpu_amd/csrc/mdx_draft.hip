@@ -114,14 +114,7 @@ __global__ __launch_bounds__(1024) void draft_row_kernel(DraftArgs a, int mode) 
             if (a.unrot) {
                 // un-rotate: the group times H256, exact in fp64, then one rounding to fp32
 #pragma unroll
-                for (int gi = 0; gi < GPW; ++gi) {
-                    double d[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) d[e] = double(v[gi][e]);
-                    fwht256_lane(d, lane);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[gi][e] = float(__dmul_rn(d[e], 0.0625));
-                }
+                for (int gi = 0; gi < GPW; ++gi) rotate256_lane(v[gi], lane);
             }
 #pragma unroll
             for (int gi = 0; gi < GPW; ++gi)
@@ -169,12 +162,9 @@ __global__ __launch_bounds__(1024) void draft_row_kernel(DraftArgs a, int mode) 
     if (a.rot == MDX_ROT_H256) {
 #pragma unroll
         for (int gi = 0; gi < GPW; ++gi) {
-            double d[4];
+            rotate256_lane(v[gi], lane);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) d[e] = double(v[gi][e]);
-            fwht256_lane(d, lane);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[gi][e] = bfround(float(__dmul_rn(d[e], 0.0625)));
+            for (int e = 0; e < 4; ++e) v[gi][e] = bfround(v[gi][e]);
         }
     }
     store_row<GPW>(a.out + row * H, G, v);

@@ -170,12 +170,9 @@ __device__ __forceinline__ void prep_row(const PrepArgs& a, const int row, float
         // fp64 FWHT, then * 1/16, rounded once to fp32 and once to bf16
 #pragma unroll
         for (int gi = 0; gi < GPW; ++gi) {
-            double d[4];
+            rotate256_lane(v[gi], lane);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) d[e] = double(v[gi][e]);
-            fwht256_lane(d, lane);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[gi][e] = bfround(float(__dmul_rn(d[e], 0.0625)));
+            for (int e = 0; e < 4; ++e) v[gi][e] = bfround(v[gi][e]);
         }
     } else if (a.rot == MDX_ROT_MATRIX) {
         // generic bf16 [256, 256] matrix: out_j = fp64 sum over k (in order, from 0.0) of the exact

@@ -37,34 +37,94 @@ __device__ __forceinline__ double h4_out(const double* a, int j) {
     return __dadd_rn(__dadd_rn(__dadd_rn(b[0], b[1]), b[2]), b[3]);
 }
 
-// fp64 fast Walsh-Hadamard transform of one 256-group held 4 elements per lane (lane l: elements
-// 4 l .. 4 l + 3): radix-4 stages along the base-4 digits of the element index (strides 1, 4, 16, 64).
-// Digit 0 is the lane's own slot, digit 1 the lane within its quad, digits 2 and 3 the quad within
-// the 16-lane row and the row; each lane computes its own output of every butterfly.
-__device__ __forceinline__ void fwht256_lane(double* d, int lane) {
-    double o[4];
+// v of this lane in the banks (quads of each row of 16) of BANKS, w of the lane that DPP control CTRL names in the
+// others' place: one v_mov_b32_dpp per 32-bit half
+template <int CTRL, int BANKS>
+__device__ __forceinline__ uint32_t dpp_banks(uint32_t v, uint32_t w) {
+    return uint32_t(__builtin_amdgcn_update_dpp(int(v), int(w), CTRL, 0xF, BANKS, false));
+}
+
+// The 4 x 4 transposition between a lane's register index r and its quad q within the row of 16: register r of
+// quad q <- register q of quad r (same lane of the quad). Two exchanges, of lane bit 3 with register bit 1 and of
+// lane bit 2 with register bit 0.
+__device__ __forceinline__ void swap_quads(uint32_t (&x)[4]) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const uint32_t a = x[r], b = x[r + 2];
+        x[r] = dpp_banks<0x128, 0xC>(a, b);      // row_ror:8
+        x[r + 2] = dpp_banks<0x128, 0x3>(b, a);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r += 2) {
+        const uint32_t a = x[r], b = x[r + 1];
+        x[r] = dpp_banks<0x114, 0xA>(a, b);      // row_shr:4
+        x[r + 1] = dpp_banks<0x104, 0x5>(b, a);  // row_shl:4
+    }
+}
+
+// The same between the register index and the row of 16 lanes: v_permlane32_swap exchanges lane bit 5 with
+// register bit 1, v_permlane16_swap lane bit 4 with register bit 0.
+__device__ __forceinline__ void swap_rows(uint32_t (&x)[4]) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const auto s = __builtin_amdgcn_permlane32_swap(x[r], x[r + 2], false, false);
+        x[r] = s[0];
+        x[r + 2] = s[1];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r += 2) {
+        const auto s = __builtin_amdgcn_permlane16_swap(x[r], x[r + 1], false, false);
+        x[r] = s[0];
+        x[r + 1] = s[1];
+    }
+}
+
+template <void (*SWAP)(uint32_t (&)[4])>
+__device__ __forceinline__ void swap_doubles(double (&d)[4]) {
+    uint32_t lo[4], hi[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, d[e]);
+        lo[e] = uint32_t(u);
+        hi[e] = uint32_t(u >> 32);
+    }
+    SWAP(lo);
+    SWAP(hi);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) d[e] = __builtin_bit_cast(double, uint64_t(lo[e]) | (uint64_t(hi[e]) << 32));
+}
+
+// H256 of one 256-group held 4 elements per lane (lane l: elements 4 l .. 4 l + 3), in place: the fp64 fast
+// Walsh-Hadamard transform times 1/16, rounded once to fp32. Radix-4 stages along the base-4 digits of the
+// element index (strides 1, 4, 16, 64): digit 0 is the lane's own register, digit 1 the lane within its quad (each
+// lane computes its own output from the quad's broadcasts), digits 2 and 3 the quad within the row of 16 lanes
+// and the row. Those two are transposed into the registers (DPP moves and lane swaps, no LDS) for a butterfly
+// inside the lane; the fp32 results go back the same way. The transposition replaces 64 ds_bpermute per group and
+// wave, which bound the transform (8 rows, row prep with rotation: K = 12288 12.0 -> 8.1 us, K = 4096 6.5 -> 5.5 us
+// per launch; without rotation 4.8 and 4.6 us).
+__device__ __forceinline__ void rotate256_lane(float (&v)[4], int lane) {
+    double d[4], o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) d[e] = double(v[e]);
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = h4_out(d, e);
-    const int j1 = lane & 3, j2 = (lane >> 2) & 3, j3 = lane >> 4;
+    const int j1 = lane & 3;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const double a[4] = {quad_lane<0>(o[e]), quad_lane<1>(o[e]), quad_lane<2>(o[e]), quad_lane<3>(o[e])};
         d[e] = h4_out(a, j1);
     }
+    swap_doubles<swap_quads>(d);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        double a[4];
+    for (int e = 0; e < 4; ++e) o[e] = h4_out(d, e);
+    swap_doubles<swap_rows>(o);
+    uint32_t f[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) a[k] = __shfl(d[e], (lane & ~12) | (k << 2), 64);
-        o[e] = h4_out(a, j2);
-    }
+    for (int e = 0; e < 4; ++e) f[e] = __float_as_uint(float(__dmul_rn(h4_out(o, e), 0.0625)));
+    swap_rows(f);
+    swap_quads(f);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        double a[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) a[k] = __shfl(o[e], (lane & 15) | (k << 4), 64);
-        d[e] = h4_out(a, j3);
-    }
+    for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(f[e]);
 }
 
 // The canonical RMSNorm factor r = 1 / sqrt(mean(x^2) + eps) of a row of K = 256 G elements held by a
