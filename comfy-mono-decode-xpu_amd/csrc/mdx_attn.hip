@@ -820,6 +820,155 @@ __global__ __launch_bounds__(D) void attn_merge_kernel(AttnArgs a) {
     a.out[(int64_t(sr) * a.H + h) * D + t] = f2bf(s > 0.f ? __fdiv_rn(o, s) : 0.f);
 }
 
+// ---- The prefill form (head_dim 64 and 128) ------------------------------------------------------
+// S consecutive rows of a chain whose K/V rows are in the cache already: row s attends tokens [0, L + s]. A unit of
+// work is (kv head, four row tiles of 16 rows in the order [16-row block][head of the group]); a wave owns one tile and
+// the four waves share the K/V stages of the streaming form (its layouts, reads and online softmax), four in flight,
+// up to the last token any of them attends. Units with the most tokens start first. One launch, no partials.
+constexpr int AP_STAGES = 4;
+
+template <int D>
+__global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
+    constexpr int KK = D / 32, DT = D / 16, STAGE = A2_STEP * 2 * D, PER = STAGE / 1024 / 4;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), g = lane >> 4, c16 = lane & 15;
+    const int tiles = (a.S + 15) / 16 * a.groups, units = (tiles + 3) / 4;
+    const int kh = blockIdx.x % a.Hk, unit = units - 1 - int(blockIdx.x) / a.Hk;
+    int L = a.seqlen[0];
+    L = L < 0 ? 0 : (L > a.cap - a.S ? a.cap - a.S : L);
+    const int x = min(unit * 4 + w, tiles - 1);  // (a tile past the last repeats it and stores nothing)
+    const bool live = unit * 4 + w < tiles;
+    const int head = kh * a.groups + x % a.groups, s0 = x / a.groups * 16;
+    const int row = min(s0 + c16, a.S - 1);
+    const int wave_end = L + min(s0 + 16, a.S);                                              // tokens of this wave's tile
+    const int end = L + min(min(unit * 4 + 3, tiles - 1) / a.groups * 16 + 16, a.S);         // of the unit
+    const int nst = (end + A2_STEP - 1) / A2_STEP;
+    u32x4 qf[KK];
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) qf[kk] = ld16(a.q + head * a.qh + row * a.qs + 32 * kk + 8 * g);
+    // the query rows have arrived before the first direct-to-LDS load goes out (see the streaming form)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qf[kk]));
+    const unsigned char* kbase = reinterpret_cast<const unsigned char*>(a.key + int64_t(kh) * a.cap * D);
+    const unsigned char* vbase = reinterpret_cast<const unsigned char*>(a.value + int64_t(kh) * a.cap * D);
+    int ktok[PER], kofs[PER], vofs[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int i = w * PER + j;
+        ktok[j] = 16 * (i & 1) + (lane >> 2);
+        kofs[j] = (4 * (i >> 1) + (lane & 3)) * 16;
+        vofs[j] = (2 * i + (lane & 1)) * 16;
+    }
+    auto issue = [&](int s_) {
+        const int s = min(s_, nst - 1);  // (past the end: the last stage again, into a free slot)
+        unsigned char* kd = smem + (s_ % AP_STAGES) * 2 * STAGE;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int o0 = (w * PER + j) * 1024;
+            const int tk = min(s * A2_STEP + ktok[j], end - 1), tv = min(s * A2_STEP + (lane >> 1), end - 1);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kbase + (tk * 2 * D + kofs[j])),
+                                             (__attribute__((address_space(3))) void*)(kd + o0), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vbase + (tv * 2 * D + vofs[j])),
+                                             (__attribute__((address_space(3))) void*)(kd + STAGE + o0), 16, 0, 0);
+        }
+    };
+    f32x4 acc[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int s = 0; s < AP_STAGES - 1; ++s) issue(s);
+    for (int s = 0; s < nst; ++s) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AP_STAGES - 2) * 2 * PER) : "memory");
+        __builtin_amdgcn_s_barrier();
+        issue(s + AP_STAGES - 1);
+        const int t0 = s * A2_STEP;
+        if (t0 >= wave_end) continue;  // (uniform in the wave: only the barriers and loads are left)
+        const unsigned char* kd = smem + (s % AP_STAGES) * 2 * STAGE;
+        u32x4 kf[2][KK];
+        stage_k<D>(kf, lds_addr(kd) + c16 * 64 + g * 16);
+        f32x4 st[2];
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            st[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk)
+                st[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[tt][kk]), as_bf16x8(qf[kk]), st[tt], 0, 0, 0);
+        }
+        u32x2 va[DT], vb2[DT];
+        stage_v<D>(va, vb2, lds_addr(kd + STAGE) + (4 * g + (c16 >> 2)) * 32 + (c16 & 3) * 8);
+        const int nvalid = L + row + 1 - t0;  // this row's tokens of the stage
+        float z[2][4], mx = -INFINITY;
+        if (__builtin_amdgcn_ballot_w64(nvalid < A2_STEP) == 0) {
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    z[tt][i] = st[tt][i] * a.zscale;
+                    mx = fmaxf(mx, z[tt][i]);
+                }
+        } else {
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    z[tt][i] = 16 * tt + 4 * g + i < nvalid ? st[tt][i] * a.zscale : -INFINITY;
+                    mx = fmaxf(mx, z[tt][i]);
+                }
+        }
+        mx = max_x32(max_x16(mx));
+        const float mnew = fmaxf(m, mx);
+        const float msub = mnew == -INFINITY ? 0.f : mnew;
+        const float alpha = __builtin_amdgcn_exp2f(m - msub);
+        float p[2][4], ps = 0.f;
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+                p[tt][i] = __builtin_amdgcn_exp2f(z[tt][i] - msub);
+                p[tt][i + 1] = __builtin_amdgcn_exp2f(z[tt][i + 1] - msub);
+                bfround2(p[tt][i], p[tt][i + 1]);
+                ps += p[tt][i];
+                ps += p[tt][i + 1];
+            }
+        ps = sum_x32(sum_x16(ps));
+        l = l * alpha + ps;
+        m = mnew;
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
+        }
+        auto top2 = [](float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); };
+        const u32x4 pf = {top2(p[0][0], p[0][1]), top2(p[0][2], p[0][3]), top2(p[1][0], p[1][1]), top2(p[1][2], p[1][3])};
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            const u32x4 vf = {va[dt].x, va[dt].y, vb2[dt].x, vb2[dt].y};
+            acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf), acc[dt], 0, 0, 0);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into this work-group's LDS may outlive it
+    if (!live || s0 + c16 >= a.S) return;
+    uint16_t* o = a.out + (int64_t(s0 + c16) * a.H + head) * D + 4 * g;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = l > 0.f ? __fdiv_rn(acc[dt][i], l) : 0.f;
+        *reinterpret_cast<uint2*>(o + 16 * dt) = make_uint2(bf16pair(v[0], v[1]), bf16pair(v[2], v[3]));
+    }
+}
+
+template <int D>
+int launch_prefill(const AttnArgs& a, hipStream_t st) {
+    constexpr size_t lds = size_t(AP_STAGES) * 2 * A2_STEP * 2 * D;
+    const int units = ((a.S + 15) / 16 * a.groups + 3) / 4;
+    allow_smem(reinterpret_cast<const void*>(&attn_prefill_kernel<D>), lds);
+    hipLaunchKernelGGL(attn_prefill_kernel<D>, dim3(unsigned(units * a.Hk)), dim3(256), lds, st, a);
+    MDX_LAUNCHED();
+    return MDX_OK;
+}
+
 // the context split's tuning (MDX_ATTN_TPW: minimum tokens per wave of a chunk; MDX_ATTN_UNITS: the
 // work-group count the chunk count aims at), read once; sweeps only
 int env_int(const char* name, int dflt, int lo, int hi) {
@@ -1046,4 +1195,33 @@ extern "C" int mdx_attn_decode_rope(const uint16_t* q, int64_t q_row_stride, int
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (stream_rtw(RT) == 2) return launch2<128, 2, 8, true>(a, st);
     return launch2<128, 4, 8, true>(a, st);
+}
+
+extern "C" int mdx_attn_prefill(const uint16_t* q, int64_t q_head_stride, int64_t q_row_stride, const uint16_t* key,
+                                const uint16_t* value, const int32_t* seqlen, uint16_t* out, int64_t H, int64_t Hk,
+                                int64_t S, int64_t D, int64_t cap, void* stream) {
+    MDX_CHECK(q && key && value && seqlen && out, "null pointer");
+    MDX_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
+    MDX_CHECK(Hk >= 1 && H % Hk == 0 && S >= 1 && S <= cap, "heads / rows within the cache");
+    MDX_CHECK(cap >= 1 && cap < (int64_t(1) << 30) / D, "cache capacity");
+    MDX_CHECK(aligned(q, 16) && aligned(key, 16) && aligned(value, 16) && aligned(out, 8) && q_head_stride % 8 == 0 &&
+                  q_row_stride % 8 == 0,
+              "16-byte aligned rows");
+    AttnArgs a{};
+    a.q = q;
+    a.qh = q_head_stride;
+    a.qs = q_row_stride;
+    a.key = key;
+    a.value = value;
+    a.seqlen = seqlen;
+    a.out = out;
+    a.H = int(H);
+    a.Hk = int(Hk);
+    a.S = int(S);
+    a.cap = int(cap);
+    a.groups = int(H / Hk);
+    a.zscale = float(1.0 / sqrt(double(D)) * 1.4426950408889634);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (D == 64) return launch_prefill<64>(a, st);
+    return launch_prefill<128>(a, st);
 }

@@ -189,13 +189,7 @@ extern "C" int mdx_bf16_linear(const uint16_t* x, const uint16_t* w, int32_t lay
     MDX_CHECK(layout == MDX_LAYOUT_ROW || layout == MDX_LAYOUT_TILE, "layout");
     MDX_CHECK(aligned(x, 16) && aligned(w, 16), "16-byte aligned x / w");
     const int tiles = int(N / 16), NC = int(K / 32);
-    // split K until about 12 waves per CU are in flight (slices must divide the chunk count)
-    int KS = 1;
-    for (int d = 1; d <= 16; ++d)
-        if (NC % d == 0) {
-            KS = d;
-            if (int64_t(tiles) * d >= 3072) break;
-        }
+    const int KS = bf16_kslices(tiles, NC);
     const int TPW = std::max(1, 4 / KS);
     Bf16Args a{x, w, residual, out, int(N), int(K), int(rows), KS, TPW, tiles, layout, 1};
     if (KS == 1 && layout == MDX_LAYOUT_TILE && NC % BF_STREAM_RING == 0 && aligned(out, 8) && !getenv("MDX_BF16_NOSTREAM")) {

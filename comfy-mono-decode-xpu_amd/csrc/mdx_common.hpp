@@ -179,6 +179,17 @@ __device__ __forceinline__ float scaleback(int32_t acc, float xs, float sc) {
 }  // namespace mdx
 
 namespace mdx {
+// The bf16 linears' K slices for `tiles` output tiles of 16 over NC 32-k chunks: K is split until about 12 waves per CU
+// are in flight (slices must divide the chunk count).
+inline int bf16_kslices(int tiles, int NC) {
+    int KS = 1;
+    for (int d = 1; d <= 16; ++d)
+        if (NC % d == 0) {
+            KS = d;
+            if (int64_t(tiles) * d >= 3072) break;
+        }
+    return KS;
+}
 // Raise a kernel's dynamic LDS limit above the 64 KiB default (gfx950 has 160 KiB per CU).
 inline void allow_smem(const void* fn, size_t bytes) {
     (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes));

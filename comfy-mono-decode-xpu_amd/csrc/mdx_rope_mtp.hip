@@ -85,7 +85,7 @@ __global__ __launch_bounds__(WAVE) void rope_kv_kernel(RopeArgs a) {
     __syncthreads();
     const int half = a.rd / 2;
     const float* f = a.freqs + s * a.fs;
-    uint16_t* dst = isq ? a.oq + (int64_t(hh) * a.S + s) * D : a.ok + (int64_t(hh) * a.S + s) * D;
+    uint16_t* dst = isq ? a.oq + (int64_t(hh) * a.S + s) * D : (a.ok ? a.ok + (int64_t(hh) * a.S + s) * D : nullptr);  // (a prefill's k: the cache only)
 #pragma unroll
     for (int j = 0; j < MAX_D / WAVE; ++j) {
         if (j >= per) continue;
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(WAVE) void rope_kv_kernel(RopeArgs a) {
             o = d < half ? rope_pair(lo, m[0], hi, m[1]) : rope_pair(hi, m[3], lo, m[2]);
         }
         const uint16_t ob = f2bf(o);
-        dst[d] = ob;
+        if (dst) dst[d] = ob;
         if (!isq && in_cache) a.key[(int64_t(hh) * a.cap + p) * D + d] = ob;
     }
 }
@@ -234,6 +234,26 @@ __global__ __launch_bounds__(256) void accept_move_kernel(MoveArgs a) {
 
 using namespace mdx;
 
+namespace {
+
+int rope_kv_run(const uint16_t* q, int64_t q_row_stride, int64_t q_head_stride, const uint16_t* k, int64_t k_row_stride,
+                int64_t k_head_stride, const uint16_t* v, int64_t v_row_stride, int64_t v_head_stride,
+                const uint16_t* weight_q, const uint16_t* weight_k, float eps_q, float eps_k, const float* freqs,
+                int64_t freqs_row_stride, uint16_t* key, uint16_t* value, const int64_t* position, uint16_t* q_out,
+                uint16_t* k_out, int64_t S, int64_t Hq, int64_t Hk, int64_t D, int64_t cap, int64_t rd, void* stream) {
+    MDX_CHECK(D >= 64 && D <= MAX_D && D % 64 == 0, "head_dim must be 64, 128, 192 or 256");
+    MDX_CHECK(rd >= 2 && rd <= D && rd % 2 == 0, "even rotary dimension in 2..head_dim");
+    MDX_CHECK(cap >= 1, "cache capacity");
+    RopeArgs a{q, k, v, q_row_stride, q_head_stride, k_row_stride, k_head_stride, v_row_stride, v_head_stride,
+               weight_q, weight_k, eps_q, eps_k, freqs, freqs_row_stride, key, value, position, q_out, k_out,
+               int(S), int(Hq), int(Hk), int(D), int(rd), int(cap)};
+    hipLaunchKernelGGL(rope_kv_kernel, dim3(unsigned(S * (Hq + 2 * Hk))), dim3(WAVE), 0, static_cast<hipStream_t>(stream), a);
+    MDX_LAUNCHED();
+    return MDX_OK;
+}
+
+}  // namespace
+
 extern "C" int mdx_qk_norm_rope_kv(const uint16_t* q, int64_t q_row_stride, int64_t q_head_stride, const uint16_t* k,
                                    int64_t k_row_stride, int64_t k_head_stride, const uint16_t* v, int64_t v_row_stride,
                                    int64_t v_head_stride, const uint16_t* weight_q, const uint16_t* weight_k,
@@ -244,16 +264,25 @@ extern "C" int mdx_qk_norm_rope_kv(const uint16_t* q, int64_t q_row_stride, int6
     MDX_CHECK(q && k && v && freqs && key && value && position && q_out && k_out, "null pointer");
     MDX_CHECK(S >= 1 && S <= 16, "1..16 rows (got %lld)", (long long)S);
     MDX_CHECK(Hq > 0 && Hk > 0 && Hq % Hk == 0, "heads");
-    MDX_CHECK(D >= 64 && D <= MAX_D && D % 64 == 0, "head_dim must be 64, 128, 192 or 256");
-    MDX_CHECK(rd >= 2 && rd <= D && rd % 2 == 0, "even rotary dimension in 2..head_dim");
-    MDX_CHECK(cap >= 1, "cache capacity");
     MDX_CHECK((weight_q == nullptr) == (weight_k == nullptr), "norm weights: both or neither");
-    RopeArgs a{q, k, v, q_row_stride, q_head_stride, k_row_stride, k_head_stride, v_row_stride, v_head_stride,
-               weight_q, weight_k, eps_q, eps_k, freqs, freqs_row_stride, key, value, position, q_out, k_out,
-               int(S), int(Hq), int(Hk), int(D), int(rd), int(cap)};
-    hipLaunchKernelGGL(rope_kv_kernel, dim3(unsigned(S * (Hq + 2 * Hk))), dim3(WAVE), 0, static_cast<hipStream_t>(stream), a);
-    MDX_LAUNCHED();
-    return MDX_OK;
+    return rope_kv_run(q, q_row_stride, q_head_stride, k, k_row_stride, k_head_stride, v, v_row_stride, v_head_stride,
+                       weight_q, weight_k, eps_q, eps_k, freqs, freqs_row_stride, key, value, position, q_out, k_out, S, Hq,
+                       Hk, D, cap, rd, stream);
+}
+
+extern "C" int mdx_prefill_rope_kv(const uint16_t* q, int64_t q_row_stride, int64_t q_head_stride, const uint16_t* k,
+                                   int64_t k_row_stride, int64_t k_head_stride, const uint16_t* v, int64_t v_row_stride,
+                                   int64_t v_head_stride, const uint16_t* weight_q, const uint16_t* weight_k,
+                                   float eps_q, float eps_k, const float* freqs, int64_t freqs_row_stride,
+                                   uint16_t* key, uint16_t* value, const int64_t* position, uint16_t* q_out,
+                                   uint16_t* k_out, int64_t S, int64_t Hq, int64_t Hk, int64_t D, int64_t cap,
+                                   int64_t rd, void* stream) {
+    MDX_CHECK(k && v && freqs && key && value && position && (Hq == 0 || (q && q_out && weight_q)) && weight_k,
+              "null pointer");
+    MDX_CHECK(S >= 1 && S <= 65535 && Hq >= 0 && Hk > 0 && Hk <= 1024 && Hq % Hk == 0 && Hq <= 1024, "rows / heads");
+    return rope_kv_run(q, q_row_stride, q_head_stride, k, k_row_stride, k_head_stride, v, v_row_stride, v_head_stride,
+                       weight_q, weight_k, eps_q, eps_k, freqs, freqs_row_stride, key, value, position, q_out, k_out, S, Hq,
+                       Hk, D, cap, rd, stream);
 }
 
 extern "C" int mdx_mtp_prep_draft(const int64_t* st, int64_t k, const float* ftab, int64_t ftab_rows, int64_t row_elems,

@@ -164,6 +164,25 @@ def stream_gemv(x, x_scale, mats, outs, gate_up=False, residuals=None, out_dtype
               _lib.ptr(silu_lut), rows, _lib.stream_of(x))
 
 
+def w4a8_gemm(x, x_scale, mats, outs, gate_up=False, residuals=None, silu_lut=None):
+    """stream_gemv for any row count (bf16 outputs): the many-row form of the W4A8 linears (mdx_w4a8_gemm)."""
+    arr = (_lib.W4P * len(mats))(*[ctypes.pointer(m.struct()) for m in mats])
+    o = (ctypes.c_void_p * len(outs))(*[t.data_ptr() for t in outs])
+    r = None
+    if residuals is not None:
+        r = (ctypes.c_void_p * len(residuals))(*[None if t is None else t.data_ptr() for t in residuals])
+    _lib.call("mdx_w4a8_gemm", _lib.ptr(x), _lib.ptr(x_scale), arr, len(mats), int(gate_up), o, r, _lib.ptr(silu_lut),
+              x.shape[0], _lib.stream_of(x))
+
+
+def bf16_gemm(x, w, out, n0=0):
+    """Columns [n0, n0 + out.shape[1]) of bf16_linear(x, w) for any row count; w tile-major bf16 [N, K], x [rows, K] and
+    out contiguous, n0 a multiple of 16."""
+    rows, K = x.shape
+    _lib.call("mdx_bf16_gemm", _lib.ptr(x), _lib.ptr(w), _lib.ptr(out), rows, w.numel() // K, n0, n0 + out.shape[1], K,
+              _lib.stream_of(x))
+
+
 def rms_rot_quant(x, norm_w, eps, rot=_lib.ROT_NONE, h=None, xn_out=None):
     K = x.shape[-1]
     rows = x.numel() // K

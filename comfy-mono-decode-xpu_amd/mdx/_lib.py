@@ -122,6 +122,20 @@ SIGNATURES = {
     "mdx_draft_silu_mul": (ctypes.c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "mdx_draft_norm_rot_quant": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, ctypes.c_float, c_int32, c_void_p,
                                                 c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
+    "mdx_w4a8_gemm_fits": (c_int32, [W4P]),
+    "mdx_w4a8_gemm": (ctypes.c_int, [c_void_p, c_void_p, ctypes.POINTER(W4P), c_int32, c_int32, ctypes.POINTER(c_void_p),
+                                     ctypes.POINTER(c_void_p), c_void_p, c_int64, c_void_p]),
+    "mdx_bf16_gemm": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64,
+                                     c_void_p]),
+    "mdx_prefill_rope_kv": (ctypes.c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64,
+                                           c_int64, c_void_p, c_void_p, ctypes.c_float, ctypes.c_float, c_void_p,
+                                           c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64,
+                                           c_int64, c_int64, c_int64, c_int64, c_void_p]),
+    "mdx_attn_prefill": (ctypes.c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
+                                        c_int64, c_int64, c_int64, c_int64, c_void_p]),
+    "mdx_gdn_run": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p,
+                                   c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_float, c_void_p,
+                                   c_void_p, c_void_p, c_int64, c_int64, c_int32, c_int64, c_int64, c_int64, c_void_p]),
     "mdx_stream_read": (ctypes.c_int, [c_void_p, c_int64, c_int32, c_void_p, c_void_p]),
     "mdx_gemv_trace": (c_int32, [c_void_p, c_int32]),
     "mdx_check_bf16_round": (ctypes.c_int, [c_void_p, c_void_p, c_void_p]),

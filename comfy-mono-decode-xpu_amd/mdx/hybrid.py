@@ -565,11 +565,104 @@ class HybridModel:
                       self.nt, self.hbuf.view(1, 1, -1), self.ctl, self.kv_ptrs, c.kv_heads, c.cap, c.head_dim,
                       self.result)
 
-    # ---- prefill (not timed) -------------------------------------------------------------------
+    # ---- prefill ---------------------------------------------------------------------------------
+    def _run_fits(self):
+        """Whether the prompt can go through the many-row kernels: the flash attention at head_dim 64 / 128, hidden
+        4096 (the row buffers of a layer), whole rotation pairs, and every W4 linear in a form the GEMM takes. The exact
+        attention and a traced prefill keep the chains, whose intermediates they are about."""
+        c = self.cfg
+        if c.attn == "exact" or _C._ATTN_MODE[0] != "fast" or self._tracing() or not c.gdn_fold:
+            return False
+        if c.head_dim not in (64, 128) or c.hidden != 4096 or self.gdn_ch % 512:
+            return False
+        return all(_lib.lib().mdx_w4a8_gemm_fits(L[r].struct()) for L in self.layers for r in L if isinstance(L[r], layout.W4))
+
+    def _mlp_run(self, x1, L, q, s, hb, q2, s2, out):
+        c, n = self.cfg, x1.shape[0]
+        st = _lib.stream_of(x1)
+        _lib.call("mdx_rms_rot_quant", _lib.ptr(x1), _lib.ptr(L["norm_post"]), float(c.eps), None, _lib.ptr(self.hrot),
+                  self.rot, _lib.ptr(q), _lib.ptr(s), n, c.hidden, st)
+        _C.w4a8_gemm(q, s, [L["g"], L["u"]], [hb], gate_up=True, silu_lut=self.silu)
+        _lib.call("mdx_rot_quant", _lib.ptr(hb), _lib.ptr(self.hrot), self.rot, _lib.ptr(q2), _lib.ptr(s2), n, hb.shape[1], st)
+        _C.w4a8_gemm(q2, s2, [L["d"]], [out], residuals=[x1])
+
+    def _prefill_run(self, tokens, nexts, tail, parity):
+        """`tokens` [n] through the layers as one run of rows, the last `tail` of them left pending in the buffers of
+        `parity` (as a verify step of those rows leaves them), and the MTP block's cache rows for all (hidden row of
+        position p with token p + 1, `nexts` [n]): the operators of the verify path, each over all n rows at once. Of the
+        MTP block only what the cache keeps is computed (fc, norm, k / v). Returns the last hidden rows."""
+        c, dev, n = self.cfg, self.dev, tokens.numel()
+        H, D, I, hv = c.hidden, c.head_dim, c.inter, c.gdn_value_heads
+        qd, kd = c.heads * D, c.kv_heads * D
+        bf = dict(dtype=torch.bfloat16, device=dev)
+        pos = torch.arange(n, dtype=torch.int64, device=dev)
+        apos = pos + self.st[0]
+        self.aseq.copy_(self.st[0:1])
+        freqs = torch.index_select(self.ftab, 0, apos)
+        x = torch.index_select(self.embed, 0, tokens)
+        x1, xn, core, z = (torch.empty(n, w, **bf) for w in (H, H, hv * 128, hv * 128))
+        proj, conv, hb = (torch.empty(n, w, **bf) for w in (self.gdn_ch, self.gdn_ch, I))
+        q1, q2 = (torch.empty(n, w, dtype=torch.int8, device=dev) for w in (max(H, qd, hv * 128), I))
+        s1, s2 = torch.empty(n, device=dev), torch.empty(n, device=dev)
+        gates = torch.empty(n, hv, 2, device=dev)
+        aq, ak, av = (torch.empty(n, w, **bf) for w in (qd, kd, kd))
+        qo, y = torch.empty(c.heads, n, D, **bf), torch.empty(n, qd, **bf)
+        st = _lib.stream_of(x)
+        p = _lib.ptr
+        for i, L in enumerate(self.layers):
+            q = q1[:, :H] if q1.shape[1] == H else q1.view(-1)[:n * H].view(n, H)
+            _lib.call("mdx_rms_rot_quant", p(x), p(L["norm_in"]), float(c.eps), p(xn), p(self.hrot), self.rot, p(q), p(s1), n,
+                      H, st)
+            if c.attention(i):
+                key, value = self.kv[i]
+                _C.w4a8_gemm(q, s1, [L["q"], L["k"], L["v"]], [aq, ak, av])
+                _lib.call("mdx_prefill_rope_kv", p(aq), qd, D, p(ak), kd, D, p(av), kd, D, p(L["qn"]), p(L["kn"]),
+                          float(c.eps), float(c.eps), p(freqs), c.rotary // 2 * 4, p(key), p(value), p(apos), p(qo), None, n,
+                          c.heads, c.kv_heads, D, c.cap, c.rotary, st)
+                _lib.call("mdx_attn_prefill", p(qo), n * D, D, p(key), p(value), p(self.aseq), p(y), c.heads, c.kv_heads, n,
+                          D, c.cap, st)
+                q = q1.view(-1)[:n * qd].view(n, qd)
+                _lib.call("mdx_rot_quant", p(y), p(self.hrot), self.rot, p(q), p(s1), n, qd, st)
+            else:
+                G = self.gdn[i]
+                _C.w4a8_gemm(q, s1, [L["qkv"], L["z"]], [proj, z])
+                _lib.call("mdx_gdn_run", p(proj), p(xn), p(L["wa"]), p(L["wb"]), H, p(L["conv_w"]), p(G["conv"]), p(G["pb"]),
+                          p(G["qb"]), p(G["gates"]), p(self.ctl), p(L["dt_bias"]), p(L["g_decay"]), p(G["rec"]), 128 ** -0.5,
+                          p(conv), p(gates), p(core), n, tail, parity, c.gdn_key_heads, hv, c.slots, st)
+                q = q1.view(-1)[:n * hv * 128].view(n, hv * 128)
+                _lib.call("mdx_gnorm_rot_quant", p(core), p(z), p(L["gnorm"]), float(c.eps), None, p(self.hrot), self.rot,
+                          p(q), p(s1), n, hv * 128, st)
+            _C.w4a8_gemm(q, s1, [L["o"]], [x1], residuals=[x])
+            self._mlp_run(x1, L, q1.view(-1)[:n * H].view(n, H), s1, hb, q2, s2, x)
+        # the MTP block's k / v rows
+        M = self.mtp
+        cat, fx, kv = torch.empty(n, 2 * H, **bf), x1, torch.empty(n, 2 * kd, **bf)
+        _C.draft_embed_norm_cat(nexts, None, None, None, self.embed, x, M["norm_e"], M["norm_h"], c.eps, c.eps, cat)
+        _C.bf16_gemm(cat, M["fc"], fx)
+        _C.draft_add_rmsnorm(fx, None, M["norm_in"], c.eps, xn)
+        _C.bf16_gemm(xn, M["qkv"], kv, n0=2 * qd)
+        mk, mv = self.mkv
+        mpos = pos + self.st[1]
+        _lib.call("mdx_prefill_rope_kv", None, 0, 0, p(kv), 2 * kd, D, p(kv[:, kd:]), 2 * kd, D, None, p(M["kn"]), float(c.eps),
+                  float(c.eps), p(freqs), c.rotary // 2 * 4, p(mk), p(mv), p(mpos), None, None, n, 0, c.kv_heads, D, c.cap,
+                  c.rotary, st)
+        self.st[0:2] += n
+        self.ctl[0:1].zero_()  # (the pending rows before the run are taken)
+        return x
+
+    RUN_ROWS = 1024  # rows of a prefill run: full GEMM tiles, 150 MB of row buffers
+
+    def _chain_ctl(self, n):
+        """The parents and the program of a chain of n rows that all commit."""
+        S = self.cfg.slots
+        return list(range(-1, n - 1)) + [-1] * (S - n) + [r | 32 for r in range(n)] + [0] * (S - n)
+
     def prefill(self, prompt):
-        """Feed prompt[:-1] through the verify path as chains of up to `slots` rows, each committed in
-        full (the next chain replays it), and the MTP block over the same chains (hidden row of
-        position p with token p + 1). The last prompt token is the first decode step's root row."""
+        """Feed prompt[:-1] through the model: as runs of many rows (_prefill_run), the rows of the last chain (up to
+        `slots` of them) left pending, which the first decode step replays; shapes the runs do not take, and prompts of
+        one chain, as chains of up to `slots` rows through the verify path, each committed in full (the next chain replays
+        it). The MTP block runs over the same rows (hidden row of position p with token p + 1). The last prompt token is
+        the first decode step's root row. Both ways leave the same state."""
         c = self.cfg
         S = c.slots
         dev = self.dev
@@ -579,10 +672,21 @@ class HybridModel:
                                f"<= the cache capacity {c.cap}")
         body = prompt[:-1]
         n0, parity = 0, 0
+        last = (body.numel() - 1) // S  # the last chain's number
+        if last > 0 and self._run_fits():
+            total, parity = body.numel(), last & 1
+            self.ctl[1:2].zero_()  # (a first chain's parity: rows pending from a decode step are replayed from the other's buffers)
+            while n0 < total:
+                n = total - n0 if total - n0 <= self.RUN_ROWS + S else self.RUN_ROWS  # (whole chains, the last with rows before it)
+                tail = total - last * S if n0 + n == total else 0
+                x = self._prefill_run(body[n0:n0 + n], prompt[n0 + 1:n0 + 1 + n], tail, parity)
+                n0 += n
+            self.hbuf.copy_(x[-1:])
+            self.ctl.copy_(torch.tensor([tail, parity] + list(range(S)) + self._chain_ctl(tail), dtype=torch.int32))
+            parity ^= 1
         while n0 < body.numel():
             n = min(S, body.numel() - n0)
-            chain_ctl = torch.tensor(list(range(-1, n - 1)) + [-1] * (S - n) + [r | 32 for r in range(n)] + [0] * (S - n),
-                                     dtype=torch.int32, device=dev)
+            chain_ctl = torch.tensor(self._chain_ctl(n), dtype=torch.int32, device=dev)
             tpos = torch.arange(n, dtype=torch.int64, device=dev)
             apos = torch.empty(n, dtype=torch.int64, device=dev)
             vpos = torch.empty(1, n, dtype=torch.int64, device=dev)

@@ -506,6 +506,54 @@ int mdx_attn_exact(const uint16_t* q, int64_t q_head_stride, int64_t q_row_strid
                    const int32_t* mask, uint16_t* out, int64_t H, int64_t Hk, int64_t S, int64_t D, int64_t cap,
                    float scale, void* stream);
 
+/* ---- many-row forms for the prompt prefill ---------------------------------------------------
+ * The reference has none (its prefill is the host framework's); these carry the decode operators' contracts to any
+ * row count, so that a prompt streams each weight once per up to 128 rows. */
+
+/* W4A8 linears of 1..65535 rows: outs[i] bf16 [rows, N_i] = mdx_stream_gemv's outputs, bit for bit (1..3 matrices
+ * sharing K, group size, scale dtype and codebook; residuals bf16 [rows, N_i] optional; gate_up: outs[0] =
+ * bf16(silu_lut[g] * u)). Weights: tile-major codes, fp16 scales in groups of at least 128 (an even number of groups)
+ * or fp8 scales (groups a multiple of 8), as mdx_w4a8_gemm_fits says. 16-byte aligned x, weights, scales and channel
+ * scales, 8-byte aligned outs / residuals. */
+int32_t mdx_w4a8_gemm_fits(const mdx_w4* w);
+int mdx_w4a8_gemm(const int8_t* x, const float* x_scale, const mdx_w4* const* mats, int32_t nmats, int32_t gate_up,
+                  uint16_t* const* outs, const uint16_t* const* residuals, const uint16_t* silu_lut, int64_t rows,
+                  void* stream);
+
+/* Columns [n0, n1) of mdx_bf16_linear's output for 1..65535 rows: out bf16 [rows, n1 - n0], w bf16 tile-major [N, K].
+ * The fp32 sums take its K slices in its order (the same bits where a slice is an even number of 32-k chunks).
+ * N, n0, n1 multiples of 16, K % 64 == 0. */
+int mdx_bf16_gemm(const uint16_t* x, const uint16_t* w, uint16_t* out, int64_t rows, int64_t N, int64_t n0, int64_t n1,
+                  int64_t K, void* stream);
+
+/* mdx_qk_norm_rope_kv for 1..65535 rows (the norm weights required); Hq == 0: only k and v (q, q_out and weight_q may
+ * be NULL); k_out may be NULL (the cache only). */
+int mdx_prefill_rope_kv(const uint16_t* q, int64_t q_row_stride, int64_t q_head_stride, const uint16_t* k,
+                        int64_t k_row_stride, int64_t k_head_stride, const uint16_t* v, int64_t v_row_stride,
+                        int64_t v_head_stride, const uint16_t* weight_q, const uint16_t* weight_k, float eps_q,
+                        float eps_k, const float* freqs, int64_t freqs_row_stride, uint16_t* key, uint16_t* value,
+                        const int64_t* position, uint16_t* q_out, uint16_t* k_out, int64_t S, int64_t Hq, int64_t Hk,
+                        int64_t D, int64_t cap, int64_t rd, void* stream);
+
+/* Causal attention of S consecutive rows whose K/V rows stand in the cache at [L, L + S), L = seqlen[0] (clamped so
+ * that L + S <= cap): row s attends tokens [0, L + s], scaled by 1/sqrt(D), P rounded to bf16, fp32 sums.
+ * out bf16 [S, H, D]. D in {64, 128}. */
+int mdx_attn_prefill(const uint16_t* q, int64_t q_head_stride, int64_t q_row_stride, const uint16_t* key,
+                     const uint16_t* value, const int32_t* seqlen, uint16_t* out, int64_t H, int64_t Hk, int64_t S,
+                     int64_t D, int64_t cap, void* stream);
+
+/* The Gated-DeltaNet core over a run of `rows` rows of a chain: after the step's pending rows (ctl: pending, parity,
+ * accepted slots; buffers of the other parity as in mdx_gdn_core), each row's conv output (qkv bf16 [rows, C]), gates
+ * (f32 [rows, HV, 2]) and raw delta-rule output (core bf16 [rows, HV * 128]). rec_state and conv_state are left after
+ * row rows - tail (at least 3 rows); the last `tail` (0..slots) rows are left pending in the buffers of tail_parity, zeros
+ * past them, as a step of those rows leaves them. Invalid control words write nothing. The caller sets ctl for the next
+ * step (tail pending rows; 0: none). */
+int mdx_gdn_run(const uint16_t* proj, const uint16_t* xn, const uint16_t* wa, const uint16_t* wb, int64_t K,
+                const uint16_t* conv_w, uint16_t* conv_state, uint16_t* proj_buf, uint16_t* qkv_buf, float* gates_buf,
+                const int32_t* ctl, const float* dt_bias, const float* g_decay, float* rec_state, float qscale,
+                uint16_t* qkv, float* gates, uint16_t* core, int64_t rows, int64_t tail, int32_t tail_parity, int64_t HK,
+                int64_t HV, int64_t slots, void* stream);
+
 /* Calibration: one streaming read of `bytes` (a multiple of 1024) from `src` with the W4A8 GEMV's load
  * pattern (1 KiB per wave instruction, four loads in flight per wave), over `work_groups` work-groups
  * of 256 threads; `sink` (4 bytes) is written only if the data hashes to a marker value. It has no
@@ -516,7 +564,7 @@ int mdx_stream_read(const void* src, int64_t bytes, int32_t work_groups, uint32_
 /* Diagnostics: the GEMV kernel variants this thread launched since the previous call (at most 64 kept),
  * as records of seven int32: [MFMA kernel (0/1), source (0 int8 rows, 1 bf16 rows quantised in the
  * prologue, 2 one row prepared in the prologue; + 4 integral decode only, + 8 per-weight 16-byte tables
- * only, + 16 per-weight 8-byte tables only), scale dtype (MDX_DT_*), rows, tiles per work-group, K
+ * only, + 16 per-weight 8-byte tables only, + 64 tables of the fp8 scale bytes only), scale dtype (MDX_DT_*), rows, tiles per work-group, K
  * slices, split-K partials kept in the table region (0/1)]. Up to max_records records are copied to out
  * (7 * max_records int32); returns how many launches were recorded, and
  * starts a new record. No counterpart in the reference: it lets tests name the decode path a shape takes. */
