@@ -8,7 +8,7 @@
 // as the reference's own kernel is not bit-identical to the chain it replaces.
 //
 // Query rows of kv head kh: r = (h % groups) * S + s for the heads h of that kv head, 16 rows per
-// row tile (rt). Both forms below compute, per 32-token step of a query row tile:
+// row tile (rt). Per 32-token step of a query row tile:
 //   S^T = K Q^T   v_mfma_f32_16x16x32_bf16, A = 16 K rows (tokens) x 32 dims, B = Q^T held in
 //                 registers; the accumulator gives each lane 4 tokens of one query row (lane % 16), so
 //                 the online softmax state of a row lives in its lanes;
@@ -19,13 +19,9 @@
 // context split is recomputed on the device from seqlen in both launches, so a captured graph
 // replays for any context length.
 //
-// The streaming form (attn2_kernel, head_dim 64 / 128): one work-group per (kv head, chunk) over all
-// of the kv head's row tiles, K/V read once from HBM into an LDS ring (see the layout note at
-// stage_k). The register form (attn_kernel, head_dim 256): work-group = (kv head, row tile, chunk) of
-// 4 waves, each owning a quarter of the chunk; K rows straight from HBM as the A operand, V transposed
-// into LDS per wave, the next step's K and V prefetched into a second register set (head_dim <= 128);
-// work-group ids dealt so that the row tiles of one (kv head, chunk) share an XCD and re-read the
-// chunk from its L2.
+// One work-group per (kv head, chunk) over all of the kv head's row tiles, K/V read once from HBM into an LDS ring (see
+// the layout note at stage_k). Head_dim 256 (4 kv heads, 8 rows of 4 heads, ctx 8192): 13.7 us per launch; with K rows
+// straight from HBM as MFMA operands, V transposed through LDS and a work-group per (row tile, chunk) it took 23.9 us.
 //
 // The tree-verify form with the Q/K prep (attn2_kernel<.., PREP>, head_dim 128): the launch also does the
 // RoPE/KV kernel's work for these rows (mdx_rope.hpp: per-head RMSNorm, split-half RoPE), so the step
@@ -36,6 +32,7 @@
 // streaming form.
 #include <math.h>
 #include <stdlib.h>
+#include <type_traits>
 
 #include "mdx_common.hpp"
 #include "mdx_rope.hpp"
@@ -48,10 +45,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int AT_WAVES = 4;
-constexpr int AT_STEP = 32;        // tokens per MFMA step
-constexpr int AT_VT_ROW = 72;      // bytes per [dim] row of the transposed V tile (64 + 8: conflict-free writes)
-constexpr int AT_MIN_TPW = 64;     // default: at least this many tokens per wave per chunk (swept: 32, 64, 128)
 constexpr float LOG2E = 1.4426950408889634f;
 
 struct AttnArgs {
@@ -67,8 +60,7 @@ struct AttnArgs {
     uint16_t* out;           // [S, H, D]
     float* part;             // [Hk][RT][C + 1][2 * 16 + 16 * D]
     int H, Hk, S, cap, groups, rows, RT, C;
-    int min_tpw;             // a chunk gives each wave at least this many tokens
-    int p2;                  // the streaming form's token parts per chunk (0: the register form)
+    int parts;               // token parts per chunk
     float zscale;            // 1/sqrt(D) * log2(e)
     // the Q/K prep (PREP launches): raw q / k rows [S][H][D] with strides (row, head), the per-head norm
     // weights (null: no norm), the rows' rotation matrices [S][rd / 2][2][2] (row stride fs floats), the
@@ -98,223 +90,7 @@ __device__ __forceinline__ u32x4 ld16(const uint16_t* p) {
     return *reinterpret_cast<const u32x4*>(p);
 }
 
-// the column of token t (0..31) in a transposed V row: lane group g's 8 k-slots are tokens
-// {4g..4g+3} (first S^T tile) and {16+4g..16+4g+3} (second tile), stored contiguously at 8g
-__device__ __forceinline__ int vt_col(int t) { return t < 16 ? 8 * (t >> 2) + (t & 3) : 8 * ((t - 16) >> 2) + 4 + (t & 3); }
-
-// per-device context split: at most C chunks of at least min_tpw tokens per wave
-__device__ __forceinline__ void split(int L, int C, int min_tpw, int& tpw, int& active) {
-    int c = (L + AT_WAVES * min_tpw - 1) / (AT_WAVES * min_tpw);
-    c = c < 1 ? 1 : (c > C ? C : c);
-    tpw = (L + AT_WAVES * c - 1) / (AT_WAVES * c);
-    tpw = (tpw + AT_STEP - 1) / AT_STEP * AT_STEP;
-    active = L > 0 ? (L + AT_WAVES * tpw - 1) / (AT_WAVES * tpw) : 0;
-}
-
-template <int D, bool PINGPONG>
-__global__ __launch_bounds__(64 * AT_WAVES) void attn_kernel(AttnArgs a) {
-    constexpr int KK = D / 32;   // MFMA k-steps over the head dim
-    constexpr int DT = D / 16;   // 16-dim output tiles
-    constexpr int NV = D / 16;   // 16-byte V loads per lane per step
-    constexpr int WREG = 72 * D; // LDS bytes per wave: the transposed V tile, later the wave's (m, l, O)
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c16 = lane & 15;
-    const int units = a.Hk * (a.C + 1);
-    const int bid = blockIdx.x;
-    const int unit = (bid % 8) + 8 * ((bid / 8) / a.RT);
-    const int rt = (bid / 8) % a.RT;
-    if (unit >= units) return;  // padding ids of the last group of 8 (not counted)
-    const int kh = unit / (a.C + 1), cslot = unit % (a.C + 1);
-    const bool tree = cslot == a.C;
-    int L = a.seqlen[0];
-    L = L < 0 ? 0 : (L > a.cap ? a.cap : L);
-    int tpw, active;
-    split(L, a.C, a.min_tpw, tpw, active);
-
-    // this lane's query row: the column of S^T and O^T it holds
-    const int r = rt * 16 + c16;
-    const bool rvalid = r < a.rows;
-    const int rr = rvalid ? r : 0;
-    const int hq = kh * a.groups + rr / a.S, sq = rr % a.S;
-    // the tree work-group of a draft launch (no mask) has no tokens and must not read the mask
-    const uint32_t rmask = (tree && rvalid && a.mask != nullptr) ? uint32_t(a.mask[sq]) : 0u;
-
-    // the wave's tokens
-    int t_begin = 0, t_end = 0;
-    const uint16_t *kb, *vb;
-    int64_t kstride, vstride;
-    if (tree) {
-        if (a.mask && w == 0) t_end = a.S;
-        kb = a.xk + kh * a.xh;
-        vb = a.xv + kh * a.vh;
-        kstride = a.xs;
-        vstride = a.vs;
-    } else {
-        if (cslot < active) {
-            t_begin = (cslot * AT_WAVES + w) * tpw;
-            t_end = min(L, t_begin + tpw);
-        }
-        kb = a.key + int64_t(kh) * a.cap * D;
-        vb = a.value + int64_t(kh) * a.cap * D;
-        kstride = vstride = D;
-    }
-
-    u32x4 qf[KK];
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk)
-        qf[kk] = rvalid ? ld16(a.q + hq * a.qh + sq * a.qs + 32 * kk + 8 * g) : u32x4{0, 0, 0, 0};
-
-    f32x4 acc[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
-    unsigned char* vt = smem + w * WREG;
-
-    // one 32-token step: S^T, online softmax, V^T through LDS, O^T
-    auto step = [&](int t0, const u32x4 (&kf)[2][KK], const u32x4 (&vr)[NV]) {
-        f32x4 st[2];
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            st[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kk = 0; kk < KK; ++kk)
-                st[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[tt][kk]), as_bf16x8(qf[kk]), st[tt], 0, 0, 0);
-        }
-        float z[2][4], mx = -INFINITY;
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int tok = t0 + 16 * tt + 4 * g + i;
-                bool ok = tok < t_end;
-                if (tree) ok = ok && ((rmask >> tok) & 1u);
-                z[tt][i] = ok ? st[tt][i] * a.zscale : -INFINITY;
-                mx = fmaxf(mx, z[tt][i]);
-            }
-        mx = max_x32(max_x16(mx));
-        const float mnew = fmaxf(m, mx);
-        const float alpha = (m == -INFINITY) ? 0.f : exp2f(m - mnew);
-        float p[2][4], ps = 0.f;
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                p[tt][i] = z[tt][i] == -INFINITY ? 0.f : bfround(exp2f(z[tt][i] - mnew));
-                ps += p[tt][i];
-            }
-        ps = sum_x32(sum_x16(ps));
-        l = l * alpha + ps;
-        m = mnew;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
-        const u32x4 pf = {bf16pair(p[0][0], p[0][1]), bf16pair(p[0][2], p[0][3]), bf16pair(p[1][0], p[1][1]),
-                          bf16pair(p[1][2], p[1][3])};
-        // V^T into LDS: tokens 2 c16 and 2 c16 + 1, dims 8 (4 jj + g) .. + 8, one dword per dim
-        const int col = 2 * vt_col(2 * c16);
-#pragma unroll
-        for (int jj = 0; jj < NV / 2; ++jj) {
-            const int d0 = 8 * (4 * jj + g);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const unsigned va = vr[2 * jj][e >> 1], vb2 = vr[2 * jj + 1][e >> 1];
-                const unsigned pr = __builtin_amdgcn_perm(vb2, va, (e & 1) ? 0x07060302u : 0x05040100u);
-                *reinterpret_cast<unsigned*>(vt + (d0 + e) * AT_VT_ROW + col) = pr;
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            const unsigned char* src = vt + (16 * dt + c16) * AT_VT_ROW + 16 * g;
-            const uint2 lo = *reinterpret_cast<const uint2*>(src), hi = *reinterpret_cast<const uint2*>(src + 8);
-            const u32x4 vf = {lo.x, lo.y, hi.x, hi.y};
-            acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf), acc[dt], 0, 0, 0);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
-    // K rows (A of S^T) and this lane's V pieces of the step at t0, clamped into the wave's range
-    // (loads past the range repeat its last token, so every load is unconditional)
-    auto load = [&](int t0, u32x4 (&kf)[2][KK], u32x4 (&vr)[NV]) {
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const int tok = max(min(t0 + 16 * tt + c16, t_end - 1), 0);
-#pragma unroll
-            for (int kk = 0; kk < KK; ++kk) kf[tt][kk] = ld16(kb + tok * kstride + 32 * kk + 8 * g);
-        }
-#pragma unroll
-        for (int j = 0; j < NV; ++j) {
-            const int tok = max(min(t0 + 2 * c16 + (j & 1), t_end - 1), 0);
-            vr[j] = ld16(vb + tok * vstride + 8 * (4 * (j >> 1) + g));
-        }
-    };
-    if (t_begin < t_end) {
-        u32x4 kA[2][KK], vA[NV];
-        load(t_begin, kA, vA);
-        if (PINGPONG) {
-            // two register sets: the next step's loads are in flight while this step computes
-            u32x4 kB[2][KK], vB[NV];
-            for (int t0 = t_begin; t0 < t_end; t0 += 2 * AT_STEP) {
-                load(t0 + AT_STEP, kB, vB);
-                step(t0, kA, vA);
-                load(t0 + 2 * AT_STEP, kA, vA);
-                if (t0 + AT_STEP < t_end) step(t0 + AT_STEP, kB, vB);
-            }
-        } else {
-            for (int t0 = t_begin; t0 < t_end; t0 += AT_STEP) {
-                if (t0 > t_begin) load(t0, kA, vA);
-                step(t0, kA, vA);
-            }
-        }
-    }
-
-    // merge the 4 waves in LDS: per wave m[16], l[16], O[16][D]
-    __syncthreads();
-    float* wr = reinterpret_cast<float*>(smem + w * WREG);
-    if (g == 0) {
-        wr[c16] = m;
-        wr[16 + c16] = l;
-    }
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4*>(wr + 32 + c16 * D + 16 * dt + 4 * g) = acc[dt];
-    __syncthreads();
-    const bool has = tree ? (a.mask != nullptr) : (cslot < active);
-    float* rec = a.part + (int64_t(kh * a.RT + rt) * (a.C + 1) + cslot) * (32 + 16 * D);
-    if (has) {
-        // the rows' maxima and the waves' weights once per row (threads 0..15), then each output
-        // element is four products; the same arithmetic, in the same order, as per element
-        __shared__ float fw[16][AT_WAVES];
-        if (threadIdx.x < 16) {
-            const int row = threadIdx.x;
-            float M = -INFINITY;
-#pragma unroll
-            for (int v = 0; v < AT_WAVES; ++v) M = fmaxf(M, reinterpret_cast<const float*>(smem + v * WREG)[row]);
-            float s = 0.f;
-#pragma unroll
-            for (int v = 0; v < AT_WAVES; ++v) {
-                const float* wv = reinterpret_cast<const float*>(smem + v * WREG);
-                const float mv = wv[row];
-                const float f = mv == -INFINITY ? 0.f : exp2f(mv - M);
-                fw[row][v] = f;
-                s += wv[16 + row] * f;
-            }
-            rec[row] = M;
-            rec[16 + row] = s;
-        }
-        __syncthreads();
-        for (int e = threadIdx.x; e < 16 * D; e += 64 * AT_WAVES) {
-            const int row = e / D, d = e % D;
-            float o = 0.f;
-#pragma unroll
-            for (int v = 0; v < AT_WAVES; ++v) o += reinterpret_cast<const float*>(smem + v * WREG)[32 + row * D + d] * fw[row][v];
-            rec[32 + e] = o;
-        }
-    }
-}
-
-// ---- The streaming form (head_dim 64 and 128) ---------------------------------------------------
+// ---- The streaming form ----------------------------------------------------------------------------
 // One work-group per (kv head, chunk): all of the kv head's query rows (up to 4 row tiles) in one
 // work-group, so each K/V byte leaves HBM once and is read from LDS by every row tile. Wave w of NWV
 // owns row tile w % RTW and token part w / RTW of the chunk (P = NWV / RTW parts; eight waves, two per
@@ -344,7 +120,17 @@ __device__ __forceinline__ uint32_t lds_addr(const unsigned char* p) {
 }
 template <int D>
 __device__ __forceinline__ void stage_k(u32x4 (&kf)[2][D / 32], uint32_t base) {
-    if constexpr (D == 128) {
+    if constexpr (D == 256) {
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+            asm volatile(
+                "ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:2048\n\tds_read_b128 %2, %8 offset:4096\n\t"
+                "ds_read_b128 %3, %8 offset:6144\n\tds_read_b128 %4, %8 offset:8192\n\tds_read_b128 %5, %8 offset:10240\n\t"
+                "ds_read_b128 %6, %8 offset:12288\n\tds_read_b128 %7, %8 offset:14336\n\ts_waitcnt lgkmcnt(0)"
+                : "=&v"(kf[tt][0]), "=&v"(kf[tt][1]), "=&v"(kf[tt][2]), "=&v"(kf[tt][3]), "=&v"(kf[tt][4]), "=&v"(kf[tt][5]),
+                  "=&v"(kf[tt][6]), "=&v"(kf[tt][7])
+                : "v"(base + tt * 1024));
+    } else if constexpr (D == 128) {
         asm volatile(
             "ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:2048\n\tds_read_b128 %2, %8 offset:4096\n\t"
             "ds_read_b128 %3, %8 offset:6144\n\tds_read_b128 %4, %8 offset:1024\n\tds_read_b128 %5, %8 offset:3072\n\t"
@@ -353,7 +139,7 @@ __device__ __forceinline__ void stage_k(u32x4 (&kf)[2][D / 32], uint32_t base) {
               "=&v"(kf[1][2]), "=&v"(kf[1][3])
             : "v"(base));
     } else {
-        static_assert(D == 64, "head_dim 64 or 128");
+        static_assert(D == 64, "head_dim 64, 128 or 256");
         asm volatile(
             "ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:2048\n\tds_read_b128 %2, %4 offset:1024\n\t"
             "ds_read_b128 %3, %4 offset:3072\n\ts_waitcnt lgkmcnt(0)"
@@ -361,23 +147,29 @@ __device__ __forceinline__ void stage_k(u32x4 (&kf)[2][D / 32], uint32_t base) {
             : "v"(base));
     }
 }
+// (dim tiles [8 H, 8 H + 8) of V into va / vb)
+template <int H, int DT>
+__device__ __forceinline__ void stage_v8(u32x2 (&va)[DT], u32x2 (&vb)[DT], uint32_t base) {
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %16\n\tds_read_b64_tr_b16 %1, %16 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %2, %16 offset:2048\n\tds_read_b64_tr_b16 %3, %16 offset:3072\n\t"
+        "ds_read_b64_tr_b16 %4, %16 offset:4096\n\tds_read_b64_tr_b16 %5, %16 offset:5120\n\t"
+        "ds_read_b64_tr_b16 %6, %16 offset:6144\n\tds_read_b64_tr_b16 %7, %16 offset:7168\n\t"
+        "ds_read_b64_tr_b16 %8, %16 offset:512\n\tds_read_b64_tr_b16 %9, %16 offset:1536\n\t"
+        "ds_read_b64_tr_b16 %10, %16 offset:2560\n\tds_read_b64_tr_b16 %11, %16 offset:3584\n\t"
+        "ds_read_b64_tr_b16 %12, %16 offset:4608\n\tds_read_b64_tr_b16 %13, %16 offset:5632\n\t"
+        "ds_read_b64_tr_b16 %14, %16 offset:6656\n\tds_read_b64_tr_b16 %15, %16 offset:7680\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(va[8 * H + 0]), "=&v"(va[8 * H + 1]), "=&v"(va[8 * H + 2]), "=&v"(va[8 * H + 3]), "=&v"(va[8 * H + 4]), "=&v"(va[8 * H + 5]), "=&v"(va[8 * H + 6]),
+          "=&v"(va[8 * H + 7]), "=&v"(vb[8 * H + 0]), "=&v"(vb[8 * H + 1]), "=&v"(vb[8 * H + 2]), "=&v"(vb[8 * H + 3]), "=&v"(vb[8 * H + 4]), "=&v"(vb[8 * H + 5]),
+          "=&v"(vb[8 * H + 6]), "=&v"(vb[8 * H + 7])
+        : "v"(base + H * 8192));
+}
 template <int D>
 __device__ __forceinline__ void stage_v(u32x2 (&va)[D / 16], u32x2 (&vb)[D / 16], uint32_t base) {
-    if constexpr (D == 128) {
-        asm volatile(
-            "ds_read_b64_tr_b16 %0, %16\n\tds_read_b64_tr_b16 %1, %16 offset:1024\n\t"
-            "ds_read_b64_tr_b16 %2, %16 offset:2048\n\tds_read_b64_tr_b16 %3, %16 offset:3072\n\t"
-            "ds_read_b64_tr_b16 %4, %16 offset:4096\n\tds_read_b64_tr_b16 %5, %16 offset:5120\n\t"
-            "ds_read_b64_tr_b16 %6, %16 offset:6144\n\tds_read_b64_tr_b16 %7, %16 offset:7168\n\t"
-            "ds_read_b64_tr_b16 %8, %16 offset:512\n\tds_read_b64_tr_b16 %9, %16 offset:1536\n\t"
-            "ds_read_b64_tr_b16 %10, %16 offset:2560\n\tds_read_b64_tr_b16 %11, %16 offset:3584\n\t"
-            "ds_read_b64_tr_b16 %12, %16 offset:4608\n\tds_read_b64_tr_b16 %13, %16 offset:5632\n\t"
-            "ds_read_b64_tr_b16 %14, %16 offset:6656\n\tds_read_b64_tr_b16 %15, %16 offset:7680\n\t"
-            "s_waitcnt lgkmcnt(0)"
-            : "=&v"(va[0]), "=&v"(va[1]), "=&v"(va[2]), "=&v"(va[3]), "=&v"(va[4]), "=&v"(va[5]), "=&v"(va[6]),
-              "=&v"(va[7]), "=&v"(vb[0]), "=&v"(vb[1]), "=&v"(vb[2]), "=&v"(vb[3]), "=&v"(vb[4]), "=&v"(vb[5]),
-              "=&v"(vb[6]), "=&v"(vb[7])
-            : "v"(base));
+    if constexpr (D >= 128) {
+        stage_v8<0>(va, vb, base);
+        if constexpr (D == 256) stage_v8<1>(va, vb, base);
     } else {
         asm volatile(
             "ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %8 offset:1024\n\t"
@@ -406,7 +198,12 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
     constexpr int STAGE = A2_STEP * RB;          // bytes of K (or V) per stage
     constexpr int NS = A2_RING / (2 * STAGE * P);  // ring stages per part
     constexpr int PER = STAGE / 1024 / RTW;      // DMA instructions per wave, stage and matrix
-    static_assert(NS >= 2 && PER >= 1 && (NS - 2) * 2 * PER <= 63, "ring geometry");
+    // A ring of two stages goes out whole in the prologue and refills a slot once every wave has read it (a second
+    // barrier per stage): filled one stage ahead, the second stage's load would go out only after the first had landed.
+    // Longer rings fill NS - 1 ahead and refill the slot of the stage before at the top of a stage.
+    constexpr bool WHOLE = NS == 2;
+    constexpr int AHEAD = WHOLE ? NS : NS - 1;  // stages issued by the prologue
+    static_assert(NS >= 2 && PER >= 1 && (AHEAD - 1) * 2 * PER <= 63, "ring geometry");
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c16 = lane & 15;
     const int rt = w % RTW, part = w / RTW;
@@ -466,7 +263,7 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
     for (int kk = 0; kk < KK; ++kk) qf[kk] = u32x4{0, 0, 0, 0};
     static_assert(!PREP || (D == 128 && NWV == 8), "the Q/K prep: head_dim 128, eight waves");
     constexpr int QROW = D + (PREP ? 8 : 0);
-    __shared__ __align__(16) uint16_t qst[64 * QROW];
+    __shared__ __align__(16) uint16_t qst[16 * RTW * QROW];
     const uint32_t qbase = lds_addr(reinterpret_cast<const unsigned char*>(qst));
     if constexpr (!PREP) {
         // part 0's wave of each row tile brings the tile's 16 rows (D / 32 loads of 1 KiB, ahead of the ring:
@@ -485,7 +282,14 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
     }
     auto read_q = [&]() {  // lane (row c16 of tile rt, k-group g): 8 elements at 32 kk + 8 g of its row
         const uint32_t ar = qbase + uint32_t((rvalid ? r : 0) * QROW + 8 * g) * 2;
-        if constexpr (KK == 4)
+        if constexpr (KK == 8)
+            asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:64\n\tds_read_b128 %2, %8 offset:128\n\t"
+                         "ds_read_b128 %3, %8 offset:192\n\tds_read_b128 %4, %8 offset:256\n\tds_read_b128 %5, %8 offset:320\n\t"
+                         "ds_read_b128 %6, %8 offset:384\n\tds_read_b128 %7, %8 offset:448\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(qf[0]), "=&v"(qf[1]), "=&v"(qf[2]), "=&v"(qf[3]), "=&v"(qf[4]), "=&v"(qf[5]), "=&v"(qf[6]),
+                           "=&v"(qf[7])
+                         : "v"(ar));
+        else if constexpr (KK == 4)
             asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:64\n\tds_read_b128 %2, %4 offset:128\n\t"
                          "ds_read_b128 %3, %4 offset:192\n\ts_waitcnt lgkmcnt(0)"
                          : "=&v"(qf[0]), "=&v"(qf[1]), "=&v"(qf[2]), "=&v"(qf[3])
@@ -538,7 +342,7 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
     float m = -INFINITY, l = 0.f;
 
     if constexpr (!PREP) {
-        for (int s = 0; s < NS - 1 && s < nst; ++s) issue(s);
+        for (int s = 0; s < AHEAD && s < nst; ++s) issue(s);
     } else {
         // The chunk work-groups issue the ring's first round, then the raw query rows (this wave's rows w,
         // w + NWV, ...; lane l: elements l and l + 64), their rotation matrices and norm weights: the wait
@@ -547,7 +351,7 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
         // load issued after them wrote, so no loaded register may be live into the stage loop: the query
         // rows go through LDS (inline asm, which the compiler does not track).
         if (!tree)
-            for (int s = 0; s < NS - 1 && s < nst; ++s) issue(s);
+            for (int s = 0; s < AHEAD && s < nst; ++s) issue(s);
         constexpr int QPW = 64 / NWV;
         float rx0[QPW], rx1[QPW];
         float4 rm[QPW];
@@ -626,8 +430,9 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
         // stage s landed (this wave's share), then everyone's share and everyone done with stage s - 1 (the
         // PREP tree stage was written to LDS before the barrier that precedes the loop: no wait)
         if (PREP && tree) {
-        } else if (s + NS - 2 < nst) {
-            __builtin_amdgcn_s_waitcnt(((((NS - 2) * 2 * PER) & 15)) | ((((NS - 2) * 2 * PER) >> 4) << 14) | (7 << 4) | (15 << 8));
+        } else if (s + AHEAD - 1 < nst) {
+            constexpr int W = (AHEAD - 1) * 2 * PER;
+            __builtin_amdgcn_s_waitcnt((W & 15) | ((W >> 4) << 14) | (7 << 4) | (15 << 8));
         } else {
             __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0): the ring's tail
         }
@@ -635,7 +440,7 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
         __builtin_amdgcn_s_barrier();
         if constexpr (!PREP)
             if (s == 0) read_q();
-        if (s + NS - 1 < nst) issue(s + NS - 1);
+        if (!WHOLE && s + NS - 1 < nst) issue(s + NS - 1);
         const unsigned char* kd = ring + (s % NS) * 2 * STAGE;
         const unsigned char* vd = kd + STAGE;
         const int t0 = t_begin + s * A2_STEP;
@@ -655,6 +460,10 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
         // of its k-slots (4 g .. 4 g + 3, then 16 + 4 g ..), the order its S^T accumulators give P^T
         u32x2 va[DT], vb2[DT];
         stage_v<D>(va, vb2, lds_addr(vd) + (4 * g + (c16 >> 2)) * 32 + (c16 & 3) * 8);
+        if (WHOLE && s + NS < nst) {  // (uniform in the work-group) this slot is read (the reads' asm ended with its wait)
+            __builtin_amdgcn_s_barrier();
+            issue(s + NS);
+        }
         // the stage's admitted tokens (bit j: token t0 + j); whole stages of the prefix skip the mask
         const int nvalid = t_end - t0;
         uint32_t mbits = nvalid >= 32 ? ~0u : (nvalid > 0 ? (1u << nvalid) - 1u : 0u);
@@ -769,55 +578,77 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
     }
 }
 
-// Merge of the chunk partials and the tree partial: one work-group per (kv head, row tile, row), one
-// thread per output dim; the partials' weights are computed once in LDS, the O loads are independent.
+// Merge of the chunk partials and the tree partial: one work-group of 256 per query row. D / 4 threads take a partial's
+// O row in 16-byte pieces, so 1024 / D groups walk the partials at once, every load issued beside the maxima (they do not
+// depend on the weights): behind the context length, one memory round trip. (One thread per dim over all partials:
+// 7.3 us per launch at 54 partials of 256, 4.5 us at 17 of 128.)
+constexpr int MERGE_T = 256;
+
 template <int D>
-__global__ __launch_bounds__(D) void attn_merge_kernel(AttnArgs a) {
-    __shared__ float wgt[72], lsum[72];
+__global__ __launch_bounds__(MERGE_T) void attn_merge_kernel(AttnArgs a) {
+    constexpr int TPR = D / 4, G = MERGE_T / TPR, PER = (65 + G - 1) / G;  // (at most 64 chunks and the tree)
+    __shared__ float wgt[PER * G];
+    __shared__ __align__(16) float osum[G][D];
     const int row = blockIdx.x % 16, rt = (blockIdx.x / 16) % a.RT, kh = blockIdx.x / (16 * a.RT);
     const int r = rt * 16 + row;
     if (r >= a.rows) return;
     int L = a.seqlen[0];
     L = L < 0 ? 0 : (L > a.cap ? a.cap : L);
-    int tpw, active;
-    if (a.p2)
-        split2(L, a.C, a.p2, tpw, active);
-    else
-        split(L, a.C, a.min_tpw, tpw, active);
+    int T, active;
+    split2(L, a.C, a.parts, T, active);
     const bool use_tree = a.mask != nullptr;
     const int np = active + (use_tree ? 1 : 0);
     const float* base = a.part + int64_t(kh * a.RT + rt) * (a.C + 1) * (32 + 16 * D);
     auto slot = [&](int i) { return i < active ? i : a.C; };
-    const int t = threadIdx.x, lane = t % 64;
-    // every wave takes the partials' maximum itself (lane i: partials i and i + 64, np <= 65), then
-    // the weights go to LDS (both waves write the same values): one barrier
-    const float m0 = lane < np ? base[slot(lane) * (32 + 16 * D) + row] : -INFINITY;
-    const float m1 = lane + 64 < np ? base[slot(lane + 64) * (32 + 16 * D) + row] : -INFINITY;
-    float M = fmaxf(m0, m1);
-    M = max_x32(max_x16(M));
-    M = fmaxf(M, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(M), 0x128, 0xF, 0xF, false)));  // row_ror:8
-    M = fmaxf(M, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(M), 0x124, 0xF, 0xF, false)));  // row_ror:4
-    M = fmaxf(M, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(M), 0x122, 0xF, 0xF, false)));  // row_ror:2
-    M = fmaxf(M, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(M), 0x121, 0xF, 0xF, false)));  // row_ror:1
-    if (t < 64 || D <= 64) {
-        if (lane < np) {
-            wgt[lane] = m0 == -INFINITY ? 0.f : exp2f(m0 - M);
-            lsum[lane] = base[slot(lane) * (32 + 16 * D) + 16 + row];
-        }
-        if (lane + 64 < np) {
-            wgt[lane + 64] = m1 == -INFINITY ? 0.f : exp2f(m1 - M);
-            lsum[lane + 64] = base[slot(lane + 64) * (32 + 16 * D) + 16 + row];
-        }
+    const int t = threadIdx.x, lane = t % 64, gi = t / TPR, d4 = (t % TPR) * 4;
+    // every wave takes the partials' maxima and sums itself (lane i: partials i and i + 64)
+    const int i0 = min(lane, max(np - 1, 0)), i1 = min(lane + 64, max(np - 1, 0));
+    float m0 = base[slot(i0) * (32 + 16 * D) + row], m1 = base[slot(i1) * (32 + 16 * D) + row];
+    const float l0 = base[slot(i0) * (32 + 16 * D) + 16 + row], l1 = base[slot(i1) * (32 + 16 * D) + 16 + row];
+    f32x4 ov[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+        ov[j] = *reinterpret_cast<const f32x4*>(base + slot(min(gi + G * j, max(np - 1, 0))) * (32 + 16 * D) + 32 + row * D + d4);
+    m0 = lane < np ? m0 : -INFINITY;
+    m1 = lane + 64 < np ? m1 : -INFINITY;
+    auto ror = [](float v, auto ctl) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctl)::value, 0xF, 0xF, false));
+    };
+    using R8 = std::integral_constant<int, 0x128>;
+    using R4 = std::integral_constant<int, 0x124>;
+    using R2 = std::integral_constant<int, 0x122>;
+    using R1 = std::integral_constant<int, 0x121>;
+    float M = max_x32(max_x16(fmaxf(m0, m1)));
+    M = fmaxf(M, ror(M, R8{}));
+    M = fmaxf(M, ror(M, R4{}));
+    M = fmaxf(M, ror(M, R2{}));
+    M = fmaxf(M, ror(M, R1{}));
+    const float w0 = m0 == -INFINITY ? 0.f : exp2f(m0 - M), w1 = m1 == -INFINITY ? 0.f : exp2f(m1 - M);
+    float s = (w0 == 0.f ? 0.f : l0 * w0) + (w1 == 0.f ? 0.f : l1 * w1);
+    s = sum_x32(sum_x16(s));
+    s += ror(s, R8{});
+    s += ror(s, R4{});
+    s += ror(s, R2{});
+    s += ror(s, R1{});
+    if (t < 64) {  // (weights past the partials are zero)
+        wgt[lane] = w0;
+        if (lane + 64 < PER * G) wgt[lane + 64] = w1;
     }
     __syncthreads();
-    float o = 0.f, s = 0.f;
-#pragma unroll 8
-    for (int i = 0; i < np; ++i) {
-        o += base[slot(i) * (32 + 16 * D) + 32 + row * D + t] * wgt[i];
-        s += lsum[i] * wgt[i];
+    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const float w = wgt[gi + G * j];
+        if (w != 0.f) o += ov[j] * w;  // (an unused record may hold anything)
     }
+    *reinterpret_cast<f32x4*>(&osum[gi][d4]) = o;
+    __syncthreads();
+    if (t >= D) return;
+    float v = osum[0][t];
+#pragma unroll
+    for (int g = 1; g < G; ++g) v += osum[g][t];
     const int h = kh * a.groups + r / a.S, sr = r % a.S;
-    a.out[(int64_t(sr) * a.H + h) * D + t] = f2bf(s > 0.f ? __fdiv_rn(o, s) : 0.f);
+    a.out[(int64_t(sr) * a.H + h) * D + t] = f2bf(s > 0.f ? __fdiv_rn(v, s) : 0.f);
 }
 
 // ---- The prefill form (head_dim 64 and 128) ------------------------------------------------------
@@ -969,34 +800,14 @@ int launch_prefill(const AttnArgs& a, hipStream_t st) {
     return MDX_OK;
 }
 
-// the context split's tuning (MDX_ATTN_TPW: minimum tokens per wave of a chunk; MDX_ATTN_UNITS: the
-// work-group count the chunk count aims at), read once; sweeps only
-int env_int(const char* name, int dflt, int lo, int hi) {
-    const char* e = getenv(name);
-    const int v = e ? atoi(e) : dflt;
-    return v < lo ? lo : (v > hi ? hi : v);
-}
-int min_tpw_default() {
-    static const int v = env_int("MDX_ATTN_TPW", AT_MIN_TPW, AT_STEP, 4096) / AT_STEP * AT_STEP;
-    return v;
-}
-int target_units() {
-    static const int v = env_int("MDX_ATTN_UNITS", 512, 8, 65536);
-    return v;
-}
-
-// the streaming form for head_dim 64 / 128 (its ring needs two stages per part; 256 does not fit),
-// unless MDX_ATTN_V1=1 (A/B sweeps only)
-bool use_stream(int D) {
-    static const int v1 = env_int("MDX_ATTN_V1", 0, 0, 1);
-    return !v1 && (D == 64 || D == 128);
-}
 int stream_rtw(int RT) { return RT <= 1 ? 1 : (RT == 2 ? 2 : 4); }
-// token parts per chunk: eight waves per work-group (two per SIMD, so one wave's LDS and MFMA waits
+// token parts per chunk (head_dim 256: a stage is 32 KiB, so two parts of two stages, or one of four with four row tiles):
+// eight waves per work-group (two per SIMD, so one wave's LDS and MFMA waits
 // overlap the other's work) where each part still gets two ring stages, else four waves (head_dim 128
 // with one row tile)
 int stream_parts(int D, int RT) {
     const int rtw = stream_rtw(RT);
+    if (D == 256) return rtw == 4 ? 1 : 2;
     if (D == 128) return rtw == 4 ? 2 : 4;
     return 8 / rtw;
 }
@@ -1011,15 +822,6 @@ int plan_chunks2(int Hk, int RT, int D, int cap, int hint) {
     return c < 1 ? 1 : (c > 64 ? 64 : c);
 }
 
-int plan_chunks(int Hk, int RT, int cap, int hint) {
-    if (hint > 0) return hint > 64 ? 64 : hint;
-    const int tpw = min_tpw_default();
-    int c = (target_units() + Hk * RT - 1) / (Hk * RT);
-    const int by_cap = (cap + AT_WAVES * tpw - 1) / (AT_WAVES * tpw);
-    c = c > by_cap ? by_cap : c;
-    return c < 1 ? 1 : (c > 64 ? 64 : c);  // the merge holds at most 64 + 1 partial weights
-}
-
 size_t workspace_bytes(int Hk, int RT, int C, int D) {
     return 256 + size_t(Hk) * RT * (C + 1) * (32 + 16 * size_t(D)) * sizeof(float);
 }
@@ -1029,31 +831,23 @@ int launch2(const AttnArgs& a, hipStream_t st) {
     allow_smem(reinterpret_cast<const void*>(&attn2_kernel<D, RTW, NWV, PREP>), A2_RING);
     hipLaunchKernelGGL((attn2_kernel<D, RTW, NWV, PREP>), dim3(a.Hk * (a.C + 1)), dim3(64 * NWV), A2_RING, st, a);
     MDX_LAUNCHED();
-    hipLaunchKernelGGL(attn_merge_kernel<D>, dim3(a.Hk * a.RT * 16), dim3(D), 0, st, a);
+    hipLaunchKernelGGL(attn_merge_kernel<D>, dim3(a.Hk * a.RT * 16), dim3(MERGE_T), 0, st, a);
     MDX_LAUNCHED();
     return MDX_OK;
 }
 
 template <int D>
 int launch(const AttnArgs& a, hipStream_t st) {
-    if (a.p2) {
-        if constexpr (D == 64 || D == 128) {
-            const int rtw = stream_rtw(a.RT);
-            if (rtw == 1) return launch2<D, 1, (D == 128 ? 4 : 8)>(a, st);
-            if (rtw == 2) return launch2<D, 2, 8>(a, st);
-            return launch2<D, 4, 8>(a, st);
-        }
+    const int rtw = stream_rtw(a.RT);
+    if constexpr (D == 256) {
+        if (rtw == 1) return launch2<D, 1, 2>(a, st);
+        if (rtw == 2) return launch2<D, 2, 4>(a, st);
+        return launch2<D, 4, 4>(a, st);
+    } else {
+        if (rtw == 1) return launch2<D, 1, (D == 128 ? 4 : 8)>(a, st);
+        if (rtw == 2) return launch2<D, 2, 8>(a, st);
+        return launch2<D, 4, 8>(a, st);
     }
-    constexpr bool PP = D <= 128;  // register ping-pong fits below 256 VGPRs up to head_dim 128
-    const int units = a.Hk * (a.C + 1);
-    const int grid = (units + 7) / 8 * 8 * a.RT;
-    const size_t lds = size_t(AT_WAVES) * 72 * D;
-    allow_smem(reinterpret_cast<const void*>(&attn_kernel<D, PP>), lds);
-    hipLaunchKernelGGL((attn_kernel<D, PP>), dim3(grid), dim3(64 * AT_WAVES), lds, st, a);
-    MDX_LAUNCHED();
-    hipLaunchKernelGGL(attn_merge_kernel<D>, dim3(a.Hk * a.RT * 16), dim3(D), 0, st, a);
-    MDX_LAUNCHED();
-    return MDX_OK;
 }
 
 }  // namespace
@@ -1064,8 +858,7 @@ using namespace mdx;
 extern "C" size_t mdx_attn_workspace(int64_t H, int64_t Hk, int64_t S, int64_t D, int64_t cap, int64_t chunks_hint) {
     if (Hk <= 0 || H % Hk != 0 || S <= 0) return 0;
     const int RT = int((H / Hk * S + 15) / 16);
-    const int C = use_stream(int(D)) ? plan_chunks2(int(Hk), RT, int(D), int(cap), int(chunks_hint))
-                                     : plan_chunks(int(Hk), RT, int(cap), int(chunks_hint));
+    const int C = plan_chunks2(int(Hk), RT, int(D), int(cap), int(chunks_hint));
     return workspace_bytes(int(Hk), RT, C, int(D));
 }
 
@@ -1086,9 +879,7 @@ extern "C" int mdx_attn_decode(const uint16_t* q, int64_t q_head_stride, int64_t
                   xk_row_stride % 8 == 0 && xv_head_stride % 8 == 0 && xv_row_stride % 8 == 0,
               "16-byte aligned rows");
     const int RT = int((H / Hk * S + 15) / 16);
-    const bool v2 = use_stream(int(D));
-    const int C = v2 ? plan_chunks2(int(Hk), RT, int(D), int(cap), int(chunks_hint))
-                     : plan_chunks(int(Hk), RT, int(cap), int(chunks_hint));
+    const int C = plan_chunks2(int(Hk), RT, int(D), int(cap), int(chunks_hint));
     MDX_CHECK(workspace && aligned(workspace, 256) && workspace_bytes_ >= workspace_bytes(int(Hk), RT, C, int(D)),
               "workspace: %zu bytes, 256-byte aligned, zeroed once", workspace_bytes(int(Hk), RT, C, int(D)));
     AttnArgs a{};
@@ -1115,8 +906,7 @@ extern "C" int mdx_attn_decode(const uint16_t* q, int64_t q_head_stride, int64_t
     a.rows = int(H / Hk * S);
     a.RT = RT;
     a.C = C;
-    a.min_tpw = chunks_hint > 0 ? AT_STEP : min_tpw_default();
-    a.p2 = v2 ? stream_parts(int(D), RT) : 0;
+    a.parts = stream_parts(int(D), RT);
     a.zscale = float(1.0 / sqrt(double(D)) * 1.4426950408889634);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (D == 64) return launch<64>(a, st);
@@ -1137,7 +927,7 @@ extern "C" int mdx_attn_decode_rope(const uint16_t* q, int64_t q_row_stride, int
                                     void* stream) {
     MDX_CHECK(q && k && v && freqs && key && value && position && seqlen && mask && k_out && out, "null pointer");
     MDX_CHECK((weight_q == nullptr) == (weight_k == nullptr), "norm weights: both or neither");
-    MDX_CHECK(D == 128 && use_stream(int(D)), "the Q/K prep form: head_dim 128 (streaming form)");
+    MDX_CHECK(D == 128, "the Q/K prep form: head_dim 128");
     MDX_CHECK(rd == 32 || rd == 64 || rd == 128, "rotary dimension 32, 64 or 128");
     MDX_CHECK(Hk >= 1 && H % Hk == 0 && S >= 1 && S <= 16, "heads / 1..16 rows");
     const int64_t rows = H / Hk * S;
@@ -1171,8 +961,7 @@ extern "C" int mdx_attn_decode_rope(const uint16_t* q, int64_t q_row_stride, int
     a.rows = int(rows);
     a.RT = RT;
     a.C = C;
-    a.min_tpw = chunks_hint > 0 ? AT_STEP : min_tpw_default();
-    a.p2 = stream_parts(int(D), RT);
+    a.parts = stream_parts(int(D), RT);
     a.zscale = float(1.0 / sqrt(double(D)) * 1.4426950408889634);
     a.rq = q;
     a.rqs = q_row_stride;

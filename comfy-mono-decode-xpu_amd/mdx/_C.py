@@ -554,10 +554,9 @@ def attn_dpas(q, key, value, seqlen, xk, xv, mask, chunks_hint=0, out=None):
 
 def rope_attn_fits(H, Hk, S, D, rd):
     """Whether qk_norm_rope_attn takes these tree-verify rows (head_dim 128, rd 32 / 64 / 128, 17..64 query
-    rows per kv head, the streaming attention form). MDX_ROPE_ATTN=0 turns the fused form off (A/B)."""
+    rows per kv head). MDX_ROPE_ATTN=0 turns the fused form off (A/B)."""
     return (_ATTN_MODE[0] != "exact" and D == 128 and rd in (32, 64, 128) and H % Hk == 0
-            and 16 < (H // Hk) * S <= 64 and os.environ.get("MDX_ATTN_V1", "0") != "1"
-            and os.environ.get("MDX_ROPE_ATTN", "1") != "0")
+            and 16 < (H // Hk) * S <= 64 and os.environ.get("MDX_ROPE_ATTN", "1") != "0")
 
 
 def qk_norm_rope_attn(rawq, rawk, vn, weightq, weightk, freqs, key, value, position, epsq, epsk, rd, seqlen, mask,

@@ -107,3 +107,11 @@ def test_attn_graph_replay_follows_device_seqlen(C, dev):
         want = ref.attention_f64(*f[:3], L, *f[3:], mask)
         got = out.float().cpu().numpy().reshape(S, H, D)
         assert np.abs(got - want).max() <= 2e-2, L
+
+
+@pytest.mark.parametrize("H,Hk,S,L", [(16, 4, 16, 127), (16, 4, 12, 129), (4, 4, 16, 6145), (8, 1, 8, 33), (16, 4, 1, 191),
+                                      (2, 1, 1, 1), (16, 4, 8, 12289)])
+def test_attn_head_dim_256_edges(C, dev, H, Hk, S, L):
+    """The streaming form at head_dim 256: one, two, three and four row tiles, contexts around its stages (32 tokens), parts
+    and the two-stage ring's refill."""
+    _case(C, dev, H, Hk, 256, L, L + 64, [-1] + [r // 2 for r in range(S - 1)], 5 + L)
