@@ -302,6 +302,7 @@ struct GemvArgs {
     int assume_int;       // MDX_DECODE_INTEGRAL (every matrix): the integral form without the check
     int pwo;              // per-wave one-shots (one int8 row, G128, assume_int): no work-group barrier
     int tbl;              // per-weight decode tables built once per work-group into LDS: 1 16-byte, 2 8-byte (gemv_table_bytes), 3 of the 256 fp8 scale bytes (SRC_B8)
+    int xg;               // SRC_XG: rows from L2
     int red_alias;        // table-only variants with int8 rows: the split-K partials reuse the table region after the loop
     int epi;
     void* out[3];
@@ -362,6 +363,9 @@ constexpr int SRC_GDN = 32;
 // 14.9 us, down 20.6 -> 10.8 us (the same matrices with fp16 ratios per 128: 13.3 and 10.0 us).
 constexpr int SRC_B8 = 64;
 constexpr int B8_BYTES = 256 * 16;
+// Added to an int8-row source of a table variant: the activation rows are not staged in LDS; each wave loads its chunks'
+// rows (16 x 128 bytes, from L2) into a ring of registers beside the weights.
+constexpr int SRC_XG = 128;
 constexpr int XP_GPW = 4;
 constexpr int HMW = 16;  // SRC_HR: maxima per lane when every wave reads them all (<= 1024 work-groups)  // SRC_XP: 256-groups per wave (K <= 1024 x waves)
 
@@ -690,10 +694,11 @@ __device__ __forceinline__ void gemv_unit(const GemvArgs& a, const int wg, const
     int g0, g1;
     unit_groups(cu0, ncu, a.lgG, ng, ESZ, g0, g1);
     const int seg = (g1 - g0) * ESZ;  // scale bytes per tile row in LDS
-    // LDS: activation rows of the K range | scales [TPW][16][seg] | reduction | parameters [128] |
-    // flag | 32 zero bytes (the activation of MFMA rows past the last)
+    // LDS: activation rows of the K range (SRC_XG: none) | scales [TPW][16][seg] |
+    // reduction | parameters [128] | flag | 32 zero bytes (the activation of MFMA rows past the last)
+    constexpr bool XG = (SRC & SRC_XG) != 0;
     uint8_t* xl = lds;
-    uint8_t* sl = xl + ((a.rows * Kr + 1023) & ~1023);
+    uint8_t* sl = xl + (((XG ? 0 : a.rows * Kr) + 1023) & ~1023);
     // (table-only variants with int8 rows may keep the split-K partials in the table region, which is dead
     // after the loop: no region of their own)
     const bool ralias = (SRC & (SRC_TBL | SRC_TBL8)) != 0 && (SRC & 3) == SRC_Q8 && a.red_alias;
@@ -749,7 +754,9 @@ __device__ __forceinline__ void gemv_unit(const GemvArgs& a, const int wg, const
                 __builtin_amdgcn_global_load_lds(ssrc + size_t(r) * ng * ESZ + (i - r * per) * 16, MDX_LDS(swv + i0 * 16), 16, 0, 0);
             }
     }
-    if (own_x && !pwo) dma_rows_to_lds(as_global(reinterpret_cast<const uint8_t*>(a.xq)) + cu0 * CHUNK_K, K, Kr, a.rows, xl, nthr);
+    static_assert(!XG || (((SRC & (SRC_TBL | SRC_TBL8 | SRC_B8)) != 0) && SRCK == SRC_Q8), "rows from L2: int8 rows, table variants");
+    static_assert(!XG || (SRC & SRC_GDN) == 0, "the Gated-DeltaNet epilogue stages its rows in the activation region");
+    if (own_x && !pwo && !XG) dma_rows_to_lds(as_global(reinterpret_cast<const uint8_t*>(a.xq)) + cu0 * CHUNK_K, K, Kr, a.rows, xl, nthr);
     for (int tsi = 0; tsi < (pwo ? 0 : a.TPW); ++tsi) {
         int tl;
         const int mm = which_mat(a, wg * a.TPW + tsi, tl);
@@ -885,8 +892,20 @@ __device__ __forceinline__ void gemv_unit(const GemvArgs& a, const int wg, const
     }
     const int last = nch > 0 ? nch - 1 : 0;
     uint4 buf[RING];
+    // SRC_XG: lane (row lane % 16, quarter kq) of the chunk's rows: its 32 k, two loads (rows past the last repeat it)
+    const MDX_G uint8_t* xg = as_global(reinterpret_cast<const uint8_t*>(a.xq)) + (XG ? min(c, a.rows - 1) * K + c0 * CHUNK_K + klane : 0);
+    uint4 xr[XG ? RING : 1][2];
+    auto load_x = [&](int p, int i) {
+        const MDX_G v4u* x4 = reinterpret_cast<const MDX_G v4u*>(xg + i * CHUNK_K);
+        const v4u u0 = x4[0], u1 = x4[1];
+        xr[p][0] = make_uint4(u0.x, u0.y, u0.z, u0.w);
+        xr[p][1] = make_uint4(u1.x, u1.y, u1.z, u1.w);
+    };
 #pragma unroll
-    for (int p = 0; p < RING; ++p) buf[p] = ldg_stream(wp + (live ? min(p, last) : 0) * wstride);
+    for (int p = 0; p < RING; ++p) {
+        buf[p] = ldg_stream(wp + (live ? min(p, last) : 0) * wstride);
+        if constexpr (XG) load_x(p, live ? min(p, last) : 0);
+    }
     const bool can_int = !a.force_exact && cbdef && (lgG >= (MFMA ? 7 : 5));
     const bool one_scale = lgG >= 5;  // (uniform) a lane's 32-k run lies in one group
     if (t == 0) *mixed = 0;
@@ -908,8 +927,9 @@ __device__ __forceinline__ void gemv_unit(const GemvArgs& a, const int wg, const
         __builtin_amdgcn_s_waitcnt((RING & 15) | ((RING >> 4) << 14) | (7 << 4) | (15 << 8));
     } else {
         // the one-shot loads (issued before the ring) are complete once at most RING loads remain
-        static_assert(RING <= 63, "vmcnt field");  // vmcnt: bits 3:0 and 15:14
-        __builtin_amdgcn_s_waitcnt((RING & 15) | ((RING >> 4) << 14) | (7 << 4) | (15 << 8));  // vmcnt(RING) only
+        constexpr int NL = XG ? 3 * RING : RING;  // (the ring's loads)
+        static_assert(NL <= 63, "vmcnt field");  // vmcnt: bits 3:0 and 15:14
+        __builtin_amdgcn_s_waitcnt((NL & 15) | ((NL >> 4) << 14) | (7 << 4) | (15 << 8));  // vmcnt(NL) only
         __builtin_amdgcn_s_waitcnt(0xC07F);                        // lgkmcnt(0): LDS writes of this wave
         __builtin_amdgcn_s_barrier();
     }
@@ -1200,9 +1220,8 @@ __device__ __forceinline__ void gemv_unit(const GemvArgs& a, const int wg, const
         v4i acc = {0, 0, 0, 0};
         const uint8_t* xrow = xl + min(lane & 15, a.rows - 1) * Kr + klane - cu0 * CHUNK_K;
         auto chunk = [&](int p, int i, bool refill) {
-            const int ch = c0 + min(i, last);
-            const uint4* x4 = reinterpret_cast<const uint4*>(xrow + ch * CHUNK_K);
-            const uint4 xa = x4[0], xb = x4[1];
+            const uint4* x4 = reinterpret_cast<const uint4*>(xrow + (c0 + min(i, last)) * CHUNK_K);
+            const uint4 xa = XG ? xr[XG ? p : 0][0] : x4[0], xb = XG ? xr[XG ? p : 0][1] : x4[1];
             const uint32_t xd[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
             uint32_t lo[4], hi[4];
             decode_tb<TB8>(buf[p], tq[p], lo, hi);
@@ -1217,6 +1236,7 @@ __device__ __forceinline__ void gemv_unit(const GemvArgs& a, const int wg, const
             }
             if (refill) {  // refill after use
                 buf[p] = ldg_stream(wp + min(i + RING, last) * wstride);
+                if constexpr (XG) load_x(p, min(i + RING, last));
                 tq[p] = tbl_of(i + RING);
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -1256,9 +1276,8 @@ __device__ __forceinline__ void gemv_unit(const GemvArgs& a, const int wg, const
         v4i acc = {0, 0, 0, 0};
         const uint8_t* xrow = xl + min(lane & 15, a.rows - 1) * Kr + klane - cu0 * CHUNK_K;
         auto chunk = [&](int p, int i, bool refill) {
-            const int ch = c0 + min(i, last);
-            const uint4* x4 = reinterpret_cast<const uint4*>(xrow + ch * CHUNK_K);
-            const uint4 xa = x4[0], xb = x4[1];
+            const uint4* x4 = reinterpret_cast<const uint4*>(xrow + (c0 + min(i, last)) * CHUNK_K);
+            const uint4 xa = XG ? xr[XG ? p : 0][0] : x4[0], xb = XG ? xr[XG ? p : 0][1] : x4[1];
             const uint32_t xd[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
             uint32_t lo[4], hi[4];
             decode_tb2(buf[p], t0[p], t1[p], lo, hi);
@@ -1273,6 +1292,7 @@ __device__ __forceinline__ void gemv_unit(const GemvArgs& a, const int wg, const
             }
             if (refill) {  // refill after use
                 buf[p] = ldg_stream(wp + min(i + RING, last) * wstride);
+                if constexpr (XG) load_x(p, min(i + RING, last));
                 t0[p] = tbl[s0[p]];
                 t1[p] = tbl[s1[p]];
                 sbytes(i + 2 * RING, s0[p], s1[p]);
@@ -1449,7 +1469,7 @@ size_t gemv_smem(const GemvArgs& a, bool mfma, int esz, int cu0, int ncu) {
         g1 = ng;
     }
     const size_t seg = size_t(g1 - g0) * esz;
-    size_t s = ((size_t(a.rows) * ncu * CHUNK_K + 1023) & ~size_t(1023)) + ((a.TPW * 16 * seg + 1023) & ~size_t(1023));
+    size_t s = (((a.xg ? size_t(0) : size_t(a.rows) * ncu * CHUNK_K) + 1023) & ~size_t(1023)) + ((a.TPW * 16 * seg + 1023) & ~size_t(1023));
     if (!a.red_alias) s += mfma ? size_t(a.TPW) * a.KS * 64 * 4 * 4 : size_t(a.TPW) * a.KS * 16 * a.rows * 4;
     s += 128 * 4 + 16 + 32;  // parameters, flag, zeros
     if (a.xp_x) s += size_t(4) * a.K;  // SRC_XP: the bf16 row and its norm weights
@@ -1508,6 +1528,7 @@ int launch_gemv_tb(const GemvArgs& a, int wgs, hipStream_t st) {
     }
     if (a.hr) return launch_gemv_h<MFMA, R, SDT, TB_RING, SRC_HR + TB>(a, wgs, st);
     if (a.xp_x) return launch_gemv_h<MFMA, R, SDT, TB_RING, SRC_XP + TB>(a, wgs, st);
+    if (a.xg) return launch_gemv_h<MFMA, R, SDT, TB_RING, SRC_Q8 + TB + SRC_XG>(a, wgs, st);
     return launch_gemv_h<MFMA, R, SDT, TB_RING, SRC_Q8 + TB>(a, wgs, st);
 }
 
@@ -1719,6 +1740,16 @@ bool gemv_gn_fits(const mdx_w4* w, int rows) {
            int64_t(rows) * (w->k / 128) <= int64_t(2) * GN_PASSES * TPW * KS;
 }
 
+// Whether a GEMV of `rows` int8 rows takes them from L2 (SRC_XG): the table variants, where the rows would not fit LDS
+// (128 KiB; they ran in two halves, each streaming the weights: 13 rows, 12288 -> 4096 9.6 + 9.6 -> 10.8 us) and the
+// tables of a work-group's tiles do (16-byte ones: at most 96 KiB). Where the rows fit, LDS is faster: its work-groups
+// share what every wave loads from L2 here (13 rows, gate/up 2 x 12288 x 4096: 14.8 against 17.0 us).
+bool xg_fits(const mdx_w4& w, int rows, bool other_src) {
+    if (rows <= 8 || int64_t(rows) * w.k <= 128 * 1024 || other_src || w.group_size < 16) return false;
+    if (w.s_dtype == MDX_DT_FP8E4M3 && w.group_size < 128) return w.k / w.group_size <= 2048;
+    return w.decode != MDX_DECODE_INTEGRAL && w.group_size >= 128 && w.k / w.group_size <= 192;
+}
+
 // Extra activation sources and outputs of one launch (all optional).
 struct GemvExtra {
     uint32_t* hmax_out = nullptr;      // EPI_SILU pair: the work-groups' |h| maxima
@@ -1747,8 +1778,10 @@ int run_gemv(const mdx_w4* const* ws, int nm, bool pair, const int8_t* xq, const
     MDX_CHECK(!ex.hmax_out || (pair && rows <= 16), "|h| maxima need a gate/up pair");
     MDX_CHECK(!ex.xp_x || (rows == 1 && gemv_xp_fits(ws, nm, pair)), "row-prep GEMV geometry");
     MDX_CHECK(!ex.gn_y || (nm == 1 && !pair && ex.gn_z && ex.gn_w && gemv_gn_fits(ws[0], rows)), "gated-norm GEMV geometry");
-    // the activation rows live in LDS: above 128 KiB, run the rows in two halves
-    if (rows > 8 && int64_t(rows) * ws[0]->k > 128 * 1024) {
+    // the table variants take many rows straight from L2 (SRC_XG); the others hold them in LDS: above 128 KiB, they run
+    // the rows in two halves
+    const bool xg = xg_fits(*ws[0], rows, ex.hr || ex.xp_x || ex.gn_y || ex.gdn);
+    if (!xg && rows > 8 && int64_t(rows) * ws[0]->k > 128 * 1024) {
         const int ra = 8, rb = rows - 8;
         int rc = run_gemv(ws, nm, pair, xq, xs, ra, epi, outs, res, out_dt, lut, st);
         if (rc) return rc;
@@ -1768,7 +1801,8 @@ int run_gemv(const mdx_w4* const* ws, int nm, bool pair, const int8_t* xq, const
                         a, total);
     if (rc) return rc;
     bool mfma = rows >= MFMA_MIN_ROWS;
-    gemv_geometry(total, a.K, pair, rows, a.TPW, a.KS);
+    gemv_geometry(total, a.K, pair, xg ? 8 : rows, a.TPW, a.KS);
+    a.xg = xg;
     a.hmax_out = ex.hmax_out;
     a.hr = ex.hr;
     a.hmax = ex.hmax;
@@ -1796,21 +1830,25 @@ int run_gemv(const mdx_w4* const* ws, int nm, bool pair, const int8_t* xq, const
         const int nw = a.TPW * a.KS;
         a.gf.nside = (rows * a.gf.HV + nw - 1) / nw;
     }
-    MDX_CHECK(gemv_smem(a, mfma, esz) <= 160 * 1024, "activation of %d rows x K=%d exceeds LDS", rows, a.K);
+    MDX_CHECK(xg || gemv_smem(a, mfma, esz) <= 160 * 1024, "activation of %d rows x K=%d exceeds LDS", rows, a.K);
     // per-weight decode tables in LDS when the scales are not asserted integral, a group spans a chunk
     // and the larger footprint still holds the grid's work-groups per CU (else fewer resident: at 8
     // rows the gate/up pair would drop from three work-groups per CU to two and lose more than the
     // tables save; there the lanes build their tables in the loop). Tables select the table-only
     // variants, which run on the MFMA kernel at every row count (at one row too: the products leave
     // the VALU to the decode).
-    if (!a.assume_int && a.lgG >= 7) {
+    const char* te = getenv("MDX_GEMV_TBL");  // MDX_GEMV_TBL=8: the 8-byte tier whenever it applies (tests)
+    const bool tbl8 = te && atoi(te) == 8 && !a.cb;
+    if (xg && a.lgG >= 7) {
+        a.tbl = tbl8 ? 2 : 1;  // (without the rows in LDS a work-group's tables always leave room for others)
+        mfma = true;
+    } else if (!a.assume_int && a.lgG >= 7) {
         const int per_cu = (wgs + 255) / 256;
         // 16-byte tables, with the split-K partials in the table region when that makes them fit (int8 rows,
         // a table region at least the partials' size); else (default codebook) 8-byte ones
         const size_t red_bytes = size_t(a.TPW) * a.KS * 64 * 4 * 4;
         const int ngr = (a.K >> a.lgG);
-        const char* te = getenv("MDX_GEMV_TBL");  // MDX_GEMV_TBL=8: the 8-byte tier whenever it applies (tests)
-        for (int tb = te && atoi(te) == 8 && !a.cb ? 2 : 1; tb <= 2; ++tb) {
+        for (int tb = tbl8 ? 2 : 1; tb <= 2; ++tb) {
             if (tb == 2 && a.cb) break;
             a.tbl = tb;
             if (int64_t(per_cu) * gemv_smem(a, true, esz) <= 160 * 1024) break;
@@ -1832,6 +1870,7 @@ int run_gemv(const mdx_w4* const* ws, int nm, bool pair, const int8_t* xq, const
         if (gemv_smem(a, true, esz) <= 160 * 1024) mfma = true;
         else a.tbl = 0;
     }
+    MDX_CHECK(!xg || (a.tbl && gemv_smem(a, true, esz) <= 160 * 1024), "rows from L2: tables within LDS");
     MDX_CHECK(!(mfma && a.xp_x) || a.tbl, "row-prep GEMV geometry (one row takes the VALU kernel or the tables)");
     // per-wave one-shots: one int8 row, caller-asserted integral scales with the default codebook,
     // G128, 16-byte runs of scales per slice and per row (MDX_GEMV_PWO=0 turns them off)
