@@ -12,9 +12,11 @@
 // the one-stage head (bf16_linear + fast_topk) whenever the exact top-n lies within the candidates.
 //
 // Launch: PK_WG work-groups of 256, each owning a contiguous segment of the vocabulary.
-//   1. candidates: the work-group's S best approximate scores (ties: the smaller index), selected as
-//      in the top-k kernel: theta = the S-th largest of the 256 thread maxima; every element >= theta
-//      belongs to a thread whose maximum is >= theta (at most S of them), then counting ranks;
+//   1. candidates: the work-group's S best approximate scores (ties: the smaller index). An element's key is
+//      32 bits, the bf16 value order above its place in the segment (at most 8192 elements). theta = the
+//      S-th largest of the maxima of the 64 quads of threads; every element >= theta belongs to a quad whose
+//      maximum is >= theta (S of them), then counting ranks. (64-bit keys and counting over 256 thread
+//      maxima: 5.2 us to theta and 1.8 us to collect, of 21 us.)
 //   2. the candidates' exact logits: int8 (the 32 candidate rows and the activation land in LDS by DMA
 //      in K blocks of 4 KiB, then v_dot4 and a wave sum per candidate; integer, so any order), bf16
 //      (the 16 candidate rows land in LDS by DMA in the MFMA
@@ -38,7 +40,7 @@ constexpr int PK_MAXN = 8;
 constexpr int PK_MAXCH = 8;
 constexpr int PK_E = 32;      // elements per thread (segments of at most 8192)
 constexpr int PK_MAXS = 32;   // candidates per work-group at most
-constexpr int PK_CAP = PK_MAXS * PK_E;
+constexpr int PK_Q = PK_T / 4;  // quads of threads
 constexpr int PK_KB = 4096;  // int8 head: K bytes per LDS block
 
 enum PickMode : int { PICK_EXACT = 0, PICK_I8 = 1, PICK_BF16 = 2 };
@@ -83,10 +85,8 @@ __device__ __forceinline__ uint64_t ld_c64(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// approximate-score selection key: the bf16 value order, then the smaller index; unique per element
-__device__ __forceinline__ uint64_t sel_key(uint16_t b, uint32_t i) {
-    return (uint64_t(key_bf16(b)) << 32) | (0xFFFFFFFFu - i);
-}
+// approximate-score selection key of place i of the segment: the bf16 value order, then the smaller index; unique
+__device__ __forceinline__ uint32_t sel_key(uint16_t b, uint32_t i) { return (uint32_t(key_bf16(b)) << 16) | (0xFFFFu - i); }
 
 // bf16 bits of a topk rank's value (inverse of key_bf16; a NaN comes back as 0x7FFF)
 __device__ __forceinline__ uint16_t bits_of_rank(uint64_t r) {
@@ -94,16 +94,32 @@ __device__ __forceinline__ uint16_t bits_of_rank(uint64_t r) {
     return uint16_t(k >= 0x8000u ? k ^ 0x8000u : k ^ 0xFFFFu);
 }
 
-__device__ __forceinline__ int count_above(const uint64_t* buf, int n, uint64_t v) {
+__device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        const uint64_t o = __shfl_xor(v, d, 64);
+        v = o > v ? o : v;
+    }
+    return v;
+}
+
+template <typename T>
+__device__ __forceinline__ int count_above(const T* buf, int n, T v) {
     int c = 0;
     for (int f0 = 0; f0 < n; f0 += 8) {
-        uint64_t x[8];
+        T x[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = buf[min(f0 + j, n - 1)];
 #pragma unroll
         for (int j = 0; j < 8; ++j) c += (f0 + j < n && x[j] > v) ? 1 : 0;
     }
     return c;
+}
+
+// the value of lane ^ 1 (CTL 0xB1) or lane ^ 2 (0x4E) of this lane's quad
+template <int CTL>
+__device__ __forceinline__ uint32_t quad_x(uint32_t v) {
+    return uint32_t(__builtin_amdgcn_mov_dpp(int(v), CTL, 0xF, 0xF, false));
 }
 
 // The bf16 lm_head kernel's MFMA chain over the candidate rows in LDS: chunk j's A operand at
@@ -124,29 +140,29 @@ __device__ __forceinline__ f32x4 pick_chain(const uint8_t* w, const uint8_t* x, 
         const int c0 = ks * NC / KS, c1 = (ks + 1) * NC / KS, cf = c0 + (c1 - c0) / PD * PD;
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
         if (cf > c0) {
-            u32x4 wv[PD], xv[PD];
-#pragma unroll
-            for (int i = 0; i < PD; ++i) {
-                wv[i] = *reinterpret_cast<const u32x4*>(w + (c0 + i) * WSTEP);
-                xv[i] = *reinterpret_cast<const u32x4*>(x + (c0 + i) * 64);
-            }
-            for (int j = c0; j < cf; j += PD) {
-                const int jn = j + PD < cf ? j + PD : j;  // the last group reads itself again (in bounds)
-                u32x4 wn[PD], xn[PD];
+            // two register sets in turn (copying the next group's operands into the current ones cost as much as its MFMAs)
+            u32x4 wA[PD], xA[PD], wB[PD], xB[PD];
+            auto load = [&](u32x4 (&wv)[PD], u32x4 (&xv)[PD], int j) {
+                const int jc = j < cf ? j : c0;  // (past the last group: any group, in bounds)
 #pragma unroll
                 for (int i = 0; i < PD; ++i) {
-                    wn[i] = *reinterpret_cast<const u32x4*>(w + (jn + i) * WSTEP);
-                    xn[i] = *reinterpret_cast<const u32x4*>(x + (jn + i) * 64);
+                    wv[i] = *reinterpret_cast<const u32x4*>(w + (jc + i) * WSTEP);
+                    xv[i] = *reinterpret_cast<const u32x4*>(x + (jc + i) * 64);
                 }
                 __builtin_amdgcn_sched_barrier(0);
+            };
+            auto run = [&](const u32x4 (&wv)[PD], const u32x4 (&xv)[PD]) {
 #pragma unroll
                 for (int i = 0; i < PD; ++i) acc = mfma(acc, wv[i], xv[i]);
                 __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < PD; ++i) {
-                    wv[i] = wn[i];
-                    xv[i] = xn[i];
-                }
+            };
+            load(wA, xA, c0);
+            for (int j = c0; j < cf; j += 2 * PD) {
+                load(wB, xB, j + PD);
+                run(wA, xA);
+                if (j + PD >= cf) break;
+                load(wA, xA, j + 2 * PD);
+                run(wB, xB);
             }
         }
         for (int j = cf; j < c1; ++j)
@@ -158,10 +174,11 @@ __device__ __forceinline__ f32x4 pick_chain(const uint8_t* w, const uint8_t* x, 
 }
 
 __global__ __launch_bounds__(PK_T) void draft_pick_kernel(PickArgs a) {
-    extern __shared__ __align__(16) uint8_t rows_lds[];  // PICK_BF16: [K / 32][64 lanes][16 B] rows, then x [K]
-    __shared__ uint64_t cand[PK_CAP];
-    __shared__ uint64_t tmax[PK_T];
-    __shared__ uint64_t theta;
+    // first the candidates (the elements of S quads at most), then PICK_BF16: [K / 32][64 lanes][16 B] rows, x [K]
+    extern __shared__ __align__(16) uint8_t rows_lds[];
+    uint32_t* cand = reinterpret_cast<uint32_t*>(rows_lds);
+    __shared__ __align__(16) uint32_t qmax[PK_Q];
+    __shared__ uint32_t theta;
     __shared__ int ncand;
     __shared__ int sel[PK_MAXS];
     __shared__ uint16_t logit[PK_MAXS];
@@ -179,34 +196,40 @@ __global__ __launch_bounds__(PK_T) void draft_pick_kernel(PickArgs a) {
     uint16_t v[PK_E];
 #pragma unroll
     for (int j = 0; j < PK_E; ++j) v[j] = a.approx[s0 + min(t + PK_T * j, len - 1)];
-    uint64_t m = 0;
+    uint32_t key[PK_E], m = 0;  // (an element past the segment: key 0, below every key)
 #pragma unroll
-    for (int j = 0; j < PK_E; ++j)
-        if (t + PK_T * j < len) {
-            const uint64_t k = sel_key(v[j], uint32_t(s0 + t + PK_T * j));
-            m = k > m ? k : m;
-        }
-    tmax[t] = m;
+    for (int j = 0; j < PK_E; ++j) {
+        key[j] = t + PK_T * j < len ? sel_key(v[j], uint32_t(t + PK_T * j)) : 0u;
+        m = max(m, key[j]);
+    }
+    m = max(m, quad_x<0xB1>(m));
+    m = max(m, quad_x<0x4E>(m));
+    if ((t & 3) == 0) qmax[t >> 2] = m;
     if (t == 0) ncand = 0;
     __syncthreads();
-    // theta: the S-th largest thread maximum (maxima are unique and every thread holds an element)
-    if (count_above(tmax, PK_T, m) == a.S - 1) theta = m;
+    // theta: the S-th largest quad maximum (maxima are unique and every thread holds an element); each thread of a quad
+    // counts the larger ones among a quarter
+    {
+        uint4 x[PK_Q / 16];
+#pragma unroll
+        for (int j = 0; j < PK_Q / 16; ++j) x[j] = reinterpret_cast<const uint4*>(qmax)[(t & 3) * (PK_Q / 16) + j];
+        uint32_t above = 0;
+#pragma unroll
+        for (int j = 0; j < PK_Q / 16; ++j) above += uint32_t(x[j].x > m) + uint32_t(x[j].y > m) + uint32_t(x[j].z > m) + uint32_t(x[j].w > m);
+        above += quad_x<0xB1>(above);
+        above += quad_x<0x4E>(above);
+        if ((t & 3) == 0 && above == uint32_t(a.S - 1)) theta = m;
+    }
     __syncthreads();
-    const uint64_t th = theta;
+    const uint32_t th = theta;
 #pragma unroll
     for (int j = 0; j < PK_E; ++j)
-        if (t + PK_T * j < len) {
-            const uint64_t k = sel_key(v[j], uint32_t(s0 + t + PK_T * j));
-            if (k >= th) {
-                const int slot = atomicAdd(&ncand, 1);
-                cand[slot] = k;  // (at most S threads hold such elements: slot < S * PK_E)
-            }
-        }
+        if (key[j] >= th) cand[atomicAdd(&ncand, 1)] = key[j];  // (S quads hold such elements: below 4 S PK_E)
     __syncthreads();
     const int nc = ncand;
     for (int i = t; i < nc; i += PK_T) {
         const int pos = count_above(cand, nc, cand[i]);
-        if (pos < a.S) sel[pos] = int(0xFFFFFFFFu - uint32_t(cand[i]));
+        if (pos < a.S) sel[pos] = int(s0) + int(0xFFFFu - (cand[i] & 0xFFFFu));
     }
     __syncthreads();
 
@@ -316,10 +339,9 @@ __global__ __launch_bounds__(PK_T) void draft_pick_kernel(PickArgs a) {
         const int pos = count_above(rk, a.S, rk[t]);
         if (pos < PK_MAXN) st_c64(a.lists + w * PK_MAXN + pos, rk[t]);
     }
-    if (t == 0) {
-        uint64_t b = 0;
-        for (int q = 0; q < a.S; ++q) b = ra[q] > b ? ra[q] : b;
-        st_c64(a.amax + w, b);
+    if (wave == 0) {
+        const uint64_t b = wave_max_u64(lane < a.S ? ra[lane] : 0);
+        if (lane == 0) st_c64(a.amax + w, b);
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -336,6 +358,7 @@ __global__ __launch_bounds__(PK_T) void draft_pick_kernel(PickArgs a) {
     if (t < PK_WG) {
         const uint64_t hd = mlist[t * PK_MAXN];
         int above = 0;
+#pragma unroll 8
         for (int q = 0; q < PK_WG; ++q) above += mlist[q * PK_MAXN] > hd ? 1 : 0;
         if (above == a.nout - 1) theta2 = hd;
     }
@@ -357,10 +380,10 @@ __global__ __launch_bounds__(PK_T) void draft_pick_kernel(PickArgs a) {
             }
         }
     }
+    uint64_t b = 0;
+    if (a.argmax_first && wave == 0) b = wave_max_u64(lane < PK_WG ? mlist[PK_WG * PK_MAXN + lane] : 0);
     if (t == 0) {
         if (a.argmax_first) {
-            uint64_t b = 0;
-            for (int q = 0; q < PK_WG; ++q) b = mlist[PK_WG * PK_MAXN + q] > b ? mlist[PK_WG * PK_MAXN + q] : b;
             const int64_t idx = int64_t(index_of<ORDER_ARGMAX>(b));
             a.token[0] = idx;
             a.vtok[a.ch[0]] = idx;
@@ -395,6 +418,7 @@ int launch_pick(PickArgs& a, const int64_t* children, int64_t nch, int64_t nvtok
         lds = (a.layout == MDX_LAYOUT_ROW && a.K % 512 == 0 ? size_t(16) * (2 * a.K + 16) : size_t(a.K / 32) * 64 * 16) +
               size_t(a.K) * 2;
     if (a.mode == PICK_I8) lds = size_t(a.S + 1) * std::min(a.K, PK_KB);
+    lds = std::max(lds, size_t(a.S) * 4 * PK_E * sizeof(uint32_t));  // the candidates
     if (lds > 64 * 1024) allow_smem(reinterpret_cast<const void*>(&draft_pick_kernel), lds);
     hipLaunchKernelGGL(draft_pick_kernel, dim3(PK_WG), dim3(PK_T), lds, st, a);
     MDX_LAUNCHED();
@@ -458,13 +482,7 @@ extern "C" int mdx_draft_pick_bf16(const uint16_t* approx, const uint16_t* x, co
     a.K = int(K);
     // the K split of mdx_bf16_linear for this shape (its chain is replayed slice by slice)
     const int tiles = int(N / 16), NC = int(K / 32);
-    int KS = 1;
-    for (int d = 1; d <= 16; ++d)
-        if (NC % d == 0) {
-            KS = d;
-            if (int64_t(tiles) * d >= 3072) break;
-        }
-    a.KS = KS;
+    a.KS = bf16_kslices(tiles, NC);
     a.nout = int(nout);
     a.argmax_first = argmax_first ? 1 : 0;
     a.top = top;
