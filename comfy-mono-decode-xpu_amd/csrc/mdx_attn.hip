@@ -80,6 +80,11 @@ struct AttnArgs {
     const int64_t* pos;
     uint16_t* k_out;
     uint16_t* q_out;
+    // the merge's output times sigmoid: out <- bf16(out * sig[gate]), gate of (row, head, d) at gate[row * gate_row + 2 D head
+    // + D + d] (the gate half of each head's 2 D projection columns); null: no gate
+    const uint16_t* gate;
+    int64_t gate_row;
+    const uint16_t* sig;
 };
 
 __device__ __forceinline__ unsigned bf16pair(float a, float b) { return unsigned(f2bf(a)) | (unsigned(f2bf(b)) << 16); }
@@ -601,6 +606,8 @@ __global__ __launch_bounds__(MERGE_T) void attn_merge_kernel(AttnArgs a) {
     const float* base = a.part + int64_t(kh * a.RT + rt) * (a.C + 1) * (32 + 16 * D);
     auto slot = [&](int i) { return i < active ? i : a.C; };
     const int t = threadIdx.x, lane = t % 64, gi = t / TPR, d4 = (t % TPR) * 4;
+    float sg = 0.f;  // (the gate's loads go out with the partials')
+    if (a.gate) sg = bf2f(a.sig[a.gate[(r % a.S) * a.gate_row + int64_t(kh * a.groups + r / a.S) * 2 * D + D + min(t, D - 1)]]);
     // every wave takes the partials' maxima and sums itself (lane i: partials i and i + 64)
     const int i0 = min(lane, max(np - 1, 0)), i1 = min(lane + 64, max(np - 1, 0));
     float m0 = base[slot(i0) * (32 + 16 * D) + row], m1 = base[slot(i1) * (32 + 16 * D) + row];
@@ -648,7 +655,9 @@ __global__ __launch_bounds__(MERGE_T) void attn_merge_kernel(AttnArgs a) {
 #pragma unroll
     for (int g = 1; g < G; ++g) v += osum[g][t];
     const int h = kh * a.groups + r / a.S, sr = r % a.S;
-    a.out[(int64_t(sr) * a.H + h) * D + t] = f2bf(s > 0.f ? __fdiv_rn(v, s) : 0.f);
+    uint16_t ob = f2bf(s > 0.f ? __fdiv_rn(v, s) : 0.f);
+    if (a.gate) ob = f2bf(__fmul_rn(bf2f(ob), sg));  // (uniform)
+    a.out[(int64_t(sr) * a.H + h) * D + t] = ob;
 }
 
 // ---- The prefill form (head_dim 64 and 128) ------------------------------------------------------
@@ -862,12 +871,13 @@ extern "C" size_t mdx_attn_workspace(int64_t H, int64_t Hk, int64_t S, int64_t D
     return workspace_bytes(int(Hk), RT, C, int(D));
 }
 
-extern "C" int mdx_attn_decode(const uint16_t* q, int64_t q_head_stride, int64_t q_row_stride, const uint16_t* key,
-                               const uint16_t* value, const int32_t* seqlen, const uint16_t* xk, int64_t xk_head_stride,
-                               int64_t xk_row_stride, const uint16_t* xv, int64_t xv_head_stride, int64_t xv_row_stride,
-                               const int32_t* mask, uint16_t* out,
-                               int64_t H, int64_t Hk, int64_t S, int64_t D, int64_t cap, int64_t chunks_hint,
-                               void* workspace, size_t workspace_bytes_, void* stream) {
+namespace {
+
+int attn_decode_run(const uint16_t* q, int64_t q_head_stride, int64_t q_row_stride, const uint16_t* key, const uint16_t* value,
+                    const int32_t* seqlen, const uint16_t* xk, int64_t xk_head_stride, int64_t xk_row_stride,
+                    const uint16_t* xv, int64_t xv_head_stride, int64_t xv_row_stride, const int32_t* mask, uint16_t* out,
+                    int64_t H, int64_t Hk, int64_t S, int64_t D, int64_t cap, int64_t chunks_hint, const uint16_t* gate,
+                    int64_t gate_row, const uint16_t* sig, void* workspace, size_t workspace_bytes_, void* stream) {
     MDX_CHECK(q && key && value && seqlen && xk && xv && out, "null pointer");
     MDX_CHECK(D == 64 || D == 128 || D == 256, "head_dim must be 64, 128 or 256");
     MDX_CHECK(Hk >= 1 && H % Hk == 0 && S >= 1 && S <= 16, "heads / 1..16 rows");
@@ -897,6 +907,9 @@ extern "C" int mdx_attn_decode(const uint16_t* q, int64_t q_head_stride, int64_t
     a.vs = xv_row_stride;
     a.mask = mask;
     a.out = out;
+    a.gate = gate;
+    a.gate_row = gate_row;
+    a.sig = sig;
     a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + 256);
     a.H = int(H);
     a.Hk = int(Hk);
@@ -912,6 +925,32 @@ extern "C" int mdx_attn_decode(const uint16_t* q, int64_t q_head_stride, int64_t
     if (D == 64) return launch<64>(a, st);
     if (D == 128) return launch<128>(a, st);
     return launch<256>(a, st);
+}
+
+}  // namespace
+
+extern "C" int mdx_attn_decode(const uint16_t* q, int64_t q_head_stride, int64_t q_row_stride, const uint16_t* key,
+                               const uint16_t* value, const int32_t* seqlen, const uint16_t* xk, int64_t xk_head_stride,
+                               int64_t xk_row_stride, const uint16_t* xv, int64_t xv_head_stride, int64_t xv_row_stride,
+                               const int32_t* mask, uint16_t* out,
+                               int64_t H, int64_t Hk, int64_t S, int64_t D, int64_t cap, int64_t chunks_hint,
+                               void* workspace, size_t workspace_bytes_, void* stream) {
+    return attn_decode_run(q, q_head_stride, q_row_stride, key, value, seqlen, xk, xk_head_stride, xk_row_stride, xv, xv_head_stride,
+                           xv_row_stride, mask, out, H, Hk, S, D, cap, chunks_hint, nullptr, 0, nullptr, workspace,
+                           workspace_bytes_, stream);
+}
+
+extern "C" int mdx_attn_decode_gated(const uint16_t* q, int64_t q_head_stride, int64_t q_row_stride, const uint16_t* key,
+                               const uint16_t* value, const int32_t* seqlen, const uint16_t* xk, int64_t xk_head_stride,
+                               int64_t xk_row_stride, const uint16_t* xv, int64_t xv_head_stride, int64_t xv_row_stride,
+                               const int32_t* mask, uint16_t* out,
+                               int64_t H, int64_t Hk, int64_t S, int64_t D, int64_t cap, int64_t chunks_hint,
+                               const uint16_t* gate, int64_t gate_row_stride, const uint16_t* sig_lut,
+                               void* workspace, size_t workspace_bytes_, void* stream) {
+    MDX_CHECK(gate && sig_lut && gate_row_stride >= 2 * H * D, "gate rows [S, >= 2 H D] and a sigmoid table");
+    return attn_decode_run(q, q_head_stride, q_row_stride, key, value, seqlen, xk, xk_head_stride, xk_row_stride, xv, xv_head_stride,
+                           xv_row_stride, mask, out, H, Hk, S, D, cap, chunks_hint, gate, gate_row_stride, sig_lut, workspace,
+                           workspace_bytes_, stream);
 }
 
 // Tree-verify attention with the RoPE/KV kernel's Q/K prep in the same launch: see the note at the top of

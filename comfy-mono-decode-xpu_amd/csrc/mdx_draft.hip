@@ -55,6 +55,17 @@ struct DraftArgs {
     int rot;        // DM_NRQ: MDX_ROT_NONE or MDX_ROT_H256
     int8_t* qx;     // DM_NRQ: int8 [rows, H] and scale [rows], or both null
     float* sx;
+    int rowq;       // DM_NRQ: the codes of the row prep (mdx_rot_quant: of bf16(v / bf16(scale))) instead of rint(v / bf16(scale))
+    // DM_EMBED with st: one more work-group does mdx_mtp_prep_draft's work (the draft's rope row, KV positions, length)
+    int64_t rows;
+    const int64_t* st;
+    int64_t depth;
+    const float* ftab;
+    int64_t cap, nf;
+    float* freqs;
+    int64_t* mpos;
+    int np;
+    int* mseq;
 };
 
 template <int GPW>
@@ -96,6 +107,14 @@ __global__ __launch_bounds__(1024) void draft_row_kernel(DraftArgs a, int mode) 
     const int64_t row = blockIdx.x;
     float v[GPW][4];
     uint2 raw[GPW], wraw[GPW];
+    if (mode == DM_EMBED && a.st && row == a.rows) {  // (uniform)
+        const int t = threadIdx.x;
+        const int64_t p = a.st[0] + a.depth, m = a.st[1] + a.depth, r = p < a.cap ? p : a.cap - 1;
+        for (int64_t i = t; i < a.nf; i += blockDim.x) a.freqs[i] = a.ftab[r * a.nf + i];
+        if (t < a.np) a.mpos[t] = m + t;
+        if (t == 0) a.mseq[0] = int(m + 1);
+        return;
+    }
     if (mode == DM_EMBED) {
         float hv[GPW][4];
         uint2 hraw[GPW], hwraw[GPW];
@@ -181,6 +200,15 @@ __global__ __launch_bounds__(1024) void draft_row_kernel(DraftArgs a, int mode) 
     const float rm = wave_max_nn(lane < W ? wmax[lane] : 0.f);
     const float s = fmaxf(__fdiv_rn(rm, 127.0f), 1e-30f);
     if (threadIdx.x == 0) a.sx[row] = s;
+    if (a.rowq) {  // (uniform)
+        const float rr = quant_rcp(s);
+#pragma unroll
+        for (int gi = 0; gi < GPW; ++gi) {
+            const int g = w + W * gi;
+            if (g < G) *reinterpret_cast<uint32_t*>(a.qx + row * H + 256 * g + 4 * lane) = quant4(v[gi], rr);
+        }
+        return;
+    }
     const float div = bf2f(f2bf(s));  // the scale in the activation dtype (never 0: s >= 1e-30)
 #pragma unroll
     for (int gi = 0; gi < GPW; ++gi) {
@@ -309,6 +337,57 @@ extern "C" int mdx_draft_norm_rot_quant(uint16_t* x, const uint16_t* h, const ui
     a.qx = qx;
     a.sx = sx;
     return launch_draft_rows(a, DM_NRQ, rows, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mdx_draft_norm_quant(uint16_t* x, const uint16_t* h, const uint16_t* w, float eps, uint16_t* xn, int8_t* qx,
+                                    float* sx, int64_t rows, int64_t H, void* stream) {
+    if (int rc = row_checks(rows, H)) return rc;
+    MDX_CHECK(x && w && xn && qx && sx, "null pointer");
+    MDX_CHECK(aligned(x, 8) && aligned(w, 8) && aligned(xn, 8) && (!h || aligned(h, 8)) && aligned(qx, 4), "aligned rows");
+    if (rows == 0) return MDX_OK;
+    DraftArgs a{};
+    a.H = int(H);
+    a.x = x;
+    a.h = h;
+    a.w = w;
+    a.eps = eps;
+    a.out = xn;
+    a.qx = qx;
+    a.sx = sx;
+    a.rowq = 1;
+    return launch_draft_rows(a, DM_NRQ, rows, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mdx_draft_embed_prep(const int64_t* token, int64_t V, const uint16_t* emb, const uint16_t* hidden,
+                                    const uint16_t* we, const uint16_t* wh, float eps_e, float eps_h, uint16_t* out, int64_t H,
+                                    const int64_t* st, int64_t k, const float* ftab, int64_t ftab_rows, int64_t row_elems,
+                                    float* freqs, int64_t* mpos, int64_t npos, int32_t* mseq, void* stream) {
+    if (int rc = row_checks(1, H)) return rc;
+    MDX_CHECK(token && emb && hidden && we && wh && out && st && ftab && freqs && mpos && mseq, "null pointer");
+    MDX_CHECK(V >= 1 && ftab_rows >= 1 && row_elems >= 1 && npos >= 0 && npos <= 64, "shapes");
+    MDX_CHECK(aligned(hidden, 8) && aligned(we, 8) && aligned(wh, 8) && aligned(out, 8) && aligned(emb, 8), "8-byte aligned rows");
+    DraftArgs a{};
+    a.H = int(H);
+    a.token = token;
+    a.V = V;
+    a.emb = emb;
+    a.hidden = hidden;
+    a.we = we;
+    a.wh = wh;
+    a.eps_e = eps_e;
+    a.eps_h = eps_h;
+    a.out = out;
+    a.rows = 1;
+    a.st = st;
+    a.depth = k;
+    a.ftab = ftab;
+    a.cap = ftab_rows;
+    a.nf = row_elems;
+    a.freqs = freqs;
+    a.mpos = mpos;
+    a.np = int(npos);
+    a.mseq = mseq;
+    return launch_draft_rows(a, DM_EMBED, 2, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mdx_draft_sigmoid_mul(const uint16_t* a, const uint16_t* qg, int64_t qg_row_stride, int64_t head_dim,

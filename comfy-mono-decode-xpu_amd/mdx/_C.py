@@ -526,6 +526,20 @@ def attn_dpas(q, key, value, seqlen, xk, xv, mask, chunks_hint=0, out=None):
     [1, S, H * D]. chunks_hint: 0 plans the context split; n > 0 caps it at n chunks per kv head."""
     if _ATTN_MODE[0] == "exact":
         return attn_exact(q, key, value, seqlen, xk, xv, mask, out)
+    return _attn_decode(q, key, value, seqlen, xk, xv, mask, chunks_hint, out)
+
+
+def attn_gated(q, key, value, seqlen, xk, xv, mask, qg, out=None):
+    """attn_dpas followed by draft_sigmoid_mul in the merge's launch: out = bf16(y * bf16(sigmoid(gate))), the gate the second
+    half of each 2 D block of the rows qg bf16 [S, >= 2 H D] (a view with a row stride). The exact attention has no such
+    form."""
+    _check(_ATTN_MODE[0] != "exact", "attn_gated: the flash attention only")
+    _check(qg.dtype == torch.bfloat16 and qg.dim() == 2 and qg.stride(1) == 1 and qg.shape[0] == q.shape[2]
+           and qg.shape[1] >= 2 * q.shape[1] * q.shape[3], "gate rows bf16 [S, >= 2 H D]")
+    return _attn_decode(q, key, value, seqlen, xk, xv, mask, 0, out, qg)
+
+
+def _attn_decode(q, key, value, seqlen, xk, xv, mask, chunks_hint, out, qg=None):
     for t, n in ((q, "q"), (key, "key"), (value, "value"), (xk, "xk"), (xv, "xv")):
         _dev(t, n)
         _check(t.dtype == torch.bfloat16 and t.dim() == 4 and t.shape[0] == 1 and t.stride(3) == 1, f"{n}: bf16 [1, ., ., D]")
@@ -545,10 +559,14 @@ def attn_dpas(q, key, value, seqlen, xk, xv, mask, chunks_hint=0, out=None):
     _check(out.dtype == torch.bfloat16 and out.is_contiguous() and out.numel() == S * H * D, "out bf16 [1, S, H * D]")
     need = _lib.lib().mdx_attn_workspace(H, Hk, S, D, cap, int(chunks_hint))
     ws = _attn_ws(q.device, need)
-    _lib.call("mdx_attn_decode", _lib.ptr(q), q.stride(1), q.stride(2), _lib.ptr(key), _lib.ptr(value), _lib.ptr(seqlen),
-              _lib.ptr(xk), xk.stride(1), xk.stride(2), _lib.ptr(xv), xv.stride(1), xv.stride(2),
-              _lib.ptr(mask) if merge else None, _lib.ptr(out),
-              H, Hk, S, D, cap, int(chunks_hint), _lib.ptr(ws), ws.numel(), _lib.stream_of(q))
+    args = (_lib.ptr(q), q.stride(1), q.stride(2), _lib.ptr(key), _lib.ptr(value), _lib.ptr(seqlen), _lib.ptr(xk),
+            xk.stride(1), xk.stride(2), _lib.ptr(xv), xv.stride(1), xv.stride(2), _lib.ptr(mask) if merge else None,
+            _lib.ptr(out), H, Hk, S, D, cap, int(chunks_hint))
+    tail = (_lib.ptr(ws), ws.numel(), _lib.stream_of(q))
+    if qg is None:
+        _lib.call("mdx_attn_decode", *args, *tail)
+    else:
+        _lib.call("mdx_attn_decode_gated", *args, _lib.ptr(qg), qg.stride(0), _lib.ptr(_luts(q.device)[0]), *tail)
     return out
 
 
@@ -1106,6 +1124,47 @@ def draft_silu_mul(gu, out):
     rows = out.numel() // I
     _, silu = _luts(gu.device)
     _lib.call("mdx_draft_silu_mul", _lib.ptr(gu), 2 * I, _lib.ptr(silu), _lib.ptr(out), rows, I, _lib.stream_of(gu))
+
+
+def bf16_gate_up(x, w, out):
+    """draft_silu_mul(bf16_linear(x, w)) in one launch: w tile-major bf16 [2 I, K] (gate rows, then up rows), out bf16
+    [rows, I], 1..16 rows (mdx_bf16_gate_up_fits(I, K))."""
+    _bf16c(x, "x")
+    _bf16c(out, "out")
+    rows, K = x.shape
+    _check(out.shape[0] == rows and w.dtype == torch.bfloat16 and w.is_contiguous() and w.numel() == 2 * out.shape[1] * K,
+           "w bf16 [2 I, K], out bf16 [rows, I]")
+    _lib.call("mdx_bf16_gate_up", _lib.ptr(x), _lib.ptr(w), _lib.ptr(_luts(x.device)[1]), _lib.ptr(out), rows, out.shape[1], K,
+              _lib.stream_of(x))
+
+
+def draft_norm_quant(x, h, w, eps, xn, qx, sx):
+    """draft_norm_rot_quant without rotation and quant_rows of its output, in one launch: x = bf16(x + h) in place, xn =
+    RMSNorm(x), qx / sx the row prep's codes and scales of xn."""
+    for t, n in ((x, "x"), (h, "h"), (w, "w"), (xn, "xn")):
+        _bf16c(t, n)
+    H = w.numel()
+    _check(x.numel() % H == 0 and h.numel() == x.numel() and xn.numel() == x.numel() and qx.numel() == x.numel()
+           and qx.dtype == torch.int8 and qx.is_contiguous() and sx.dtype == torch.float32 and sx.is_contiguous()
+           and sx.numel() == x.numel() // H, "x / h / xn bf16, qx int8 [rows, H], sx float [rows]")
+    _lib.call("mdx_draft_norm_quant", _lib.ptr(x), _lib.ptr(h), _lib.ptr(w), float(eps), _lib.ptr(xn), _lib.ptr(qx),
+              _lib.ptr(sx), x.numel() // H, H, _lib.stream_of(x))
+
+
+def draft_embed_prep(token, emb, hidden, we, wh, eps_e, eps_h, out, st, k, ftab, freqs, mpos, mseq):
+    """draft_embed_norm_cat of one row (token int64 [1] of the bf16 table emb) and mtp_prep_draft, in one launch."""
+    for t, n in ((emb, "emb"), (hidden, "hidden"), (we, "we"), (wh, "wh"), (out, "out")):
+        _bf16c(t, n)
+    _i64(token, "token")
+    _i64(st, "st")
+    _i64(mpos, "mtp position")
+    H, n, cap = we.numel(), freqs.numel(), ftab.shape[2]
+    _check(token.numel() == 1 and emb.shape[1] == H and hidden.numel() == H and out.numel() == 2 * H, "one row")
+    _check(mseq.dtype == torch.int32 and ftab.dtype == torch.float32 and ftab.is_contiguous() and freqs.dtype == torch.float32
+           and freqs.is_contiguous() and ftab.numel() == cap * n, "rope table [.., .., cap, ...] / row float")
+    _lib.call("mdx_draft_embed_prep", _lib.ptr(token), emb.shape[0], _lib.ptr(emb), _lib.ptr(hidden), _lib.ptr(we), _lib.ptr(wh),
+              float(eps_e), float(eps_h), _lib.ptr(out), H, _lib.ptr(st), int(k), _lib.ptr(ftab), cap, n, _lib.ptr(freqs),
+              _lib.ptr(mpos), mpos.numel(), _lib.ptr(mseq), _lib.stream_of(st))
 
 
 def draft_norm_rot_quant(x, h, w, eps, hmat, xr, qx, sx):

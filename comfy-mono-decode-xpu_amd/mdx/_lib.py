@@ -122,6 +122,17 @@ SIGNATURES = {
     "mdx_draft_silu_mul": (ctypes.c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "mdx_draft_norm_rot_quant": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, ctypes.c_float, c_int32, c_void_p,
                                                 c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
+    "mdx_attn_decode_gated": (ctypes.c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
+                                             c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64,
+                                             c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
+                                             c_size_t, c_void_p]),
+    "mdx_bf16_gate_up_fits": (c_int32, [c_int64, c_int64]),
+    "mdx_bf16_gate_up": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p]),
+    "mdx_draft_norm_quant": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, ctypes.c_float, c_void_p, c_void_p, c_void_p,
+                                            c_int64, c_int64, c_void_p]),
+    "mdx_draft_embed_prep": (ctypes.c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_float,
+                                            ctypes.c_float, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64,
+                                            c_void_p, c_void_p, c_int64, c_void_p, c_void_p]),
     "mdx_w4a8_gemm_fits": (c_int32, [W4P]),
     "mdx_w4a8_gemm": (ctypes.c_int, [c_void_p, c_void_p, ctypes.POINTER(W4P), c_int32, c_int32, ctypes.POINTER(c_void_p),
                                      ctypes.POINTER(c_void_p), c_void_p, c_int64, c_void_p]),

@@ -405,18 +405,26 @@ class HybridModel:
                 self._gdn_layer(i, x, R)
             self._tr(f"L{i}.out", x)
 
-    def mtp_block(self, n, tok, h, freqs, kvpos, seq, mask):
+    def mtp_block(self, n, tok, h, freqs, kvpos, seq, mask, depth=None):
         """The MTP block over n rows (tokens `tok` [n], hidden rows `h` [n, H]), in the fused-op structure
         of comfy_mono_decode_xpu/draft_head.py:179-212: cat(RMSNorm_e(embed[tok]), RMSNorm_h(h)) -> fc -> x;
         RMSNorm_in -> q|gate, k, v -> Q/K norm + RoPE + the MTP KV write at kvpos -> attention over the MTP
         cache prefix [0, seq) (and, with a mask, the block's own rows) -> times sigmoid(gate) -> o_proj;
         x += o, RMSNorm_post -> gate|up -> SiLU(gate) * up -> down; x += down, RMSNorm_f. Leaves the new
-        hidden rows x in self.dh[:n] and their final norm (the lm_head input) in self.dxf[:n]."""
+        hidden rows x in self.dh[:n] and their final norm (the lm_head input) in self.dxf[:n]; for the two-stage
+        draft head of a bf16 lm_head also its int8 row in self.dqx / self.dsx. depth: one draft row at that depth, the
+        step's positions (mtp_prep_draft) stored by the first launch. A traced step takes the elementwise ops as launches
+        of their own (their inputs are in the trace)."""
         c, M = self.cfg, self.mtp
         H, D = c.hidden, c.head_dim
         qd, kd = c.heads * D, c.kv_heads * D
+        fused = not self._tracing()
         cat = _C._buf(self.dcat, n, 2 * H)
-        _C.draft_embed_norm_cat(tok.view(-1), None, None, None, self.embed, h, M["norm_e"], M["norm_h"], c.eps, c.eps, cat)
+        if depth is None:
+            _C.draft_embed_norm_cat(tok.view(-1), None, None, None, self.embed, h, M["norm_e"], M["norm_h"], c.eps, c.eps, cat)
+        else:
+            _C.draft_embed_prep(tok.view(-1), self.embed, h, M["norm_e"], M["norm_h"], c.eps, c.eps, cat, self.st, depth,
+                                self.ftab.view(1, 1, c.cap, c.rotary // 2, 2, 2), self.dfreqs, self.mpos, self.mseq)
         x = _C._buf(self.dh, n, H)
         xn = _C._buf(self.dxn, n, H)
         _C.bf16_linear(cat, M["fc"], out=x)
@@ -435,14 +443,17 @@ class HybridModel:
         qo = torch.empty(1, c.heads, n, D, dtype=torch.bfloat16, device=self.dev)
         ko = torch.empty(1, c.kv_heads, n, D, dtype=torch.bfloat16, device=self.dev)
         _C.qk_norm_rope_kv(qv, kv_, vv, M["qn"], M["kn"], freqs, mk, mv, kvpos, c.eps, c.eps, c.rotary, outs=(qo, ko))
-        y = _C._buf(self.dy, n, qd)
-        self._attend(qo, mk, mv, seq, ko, vv.transpose(1, 2), self.empty_mask if mask is None else mask,
-                     y.view(1, n, qd))
         gy = _C._buf(self.dgy, n, qd)
-        _C.draft_sigmoid_mul(y, qg if n > 1 else qg.view(-1), D, gy)
+        mask = self.empty_mask if mask is None else mask
+        if fused and c.attn != "exact" and _C._ATTN_MODE[0] != "exact":
+            _C.attn_gated(qo, mk, mv, seq, ko, vv.transpose(1, 2), mask, qg, out=gy.view(1, n, qd))
+        else:
+            y = _C._buf(self.dy, n, qd)
+            self._attend(qo, mk, mv, seq, ko, vv.transpose(1, 2), mask, y.view(1, n, qd))
+            _C.draft_sigmoid_mul(y, qg if n > 1 else qg.view(-1), D, gy)
+            self._tr("mtp.y", y)
         self._tr("mtp.qo", qo)
         self._tr("mtp.ko", ko)
-        self._tr("mtp.y", y)
         self._tr("mtp.gy", gy)
         o = _C._buf(self.do, n, H)
         _C.bf16_linear(gy, M["o"], out=o)
@@ -450,13 +461,16 @@ class HybridModel:
         _C.draft_add_rmsnorm(x, o, M["norm_post"], c.eps, xn)
         self._tr("mtp.x_post", x)
         self._tr("mtp.xn_post", xn)
-        gu = _C._buf(self.dgu, n, 2 * c.inter)
-        _C.bf16_linear(xn, M["gu"], out=gu)
         act = _C._buf(self.dact, n, c.inter)
-        _C.draft_silu_mul(gu, act)
+        if fused and _lib.lib().mdx_bf16_gate_up_fits(c.inter, H):
+            _C.bf16_gate_up(xn, M["gu"], act)
+        else:
+            gu = _C._buf(self.dgu, n, 2 * c.inter)
+            _C.bf16_linear(xn, M["gu"], out=gu)
+            _C.draft_silu_mul(gu, act)
+            self._tr("mtp.gu", gu)
         d = _C._buf(self.dd, n, H)
         _C.bf16_linear(act, M["d"], out=d)
-        self._tr("mtp.gu", gu)
         self._tr("mtp.act", act)
         self._tr("mtp.d", d)
         if c.head == "int8":
@@ -465,6 +479,8 @@ class HybridModel:
                                     self.dsx[:n])
             self._tr("mtp.qx", self.dqx[:n])
             self._tr("mtp.sx", self.dsx[:n])
+        elif c.two_stage:
+            _C.draft_norm_quant(x, d, M["norm_f"], c.eps, _C._buf(self.dxf, n, H), self.dqx[:n], self.dsx[:n])
         else:
             _C.draft_norm_rot_quant(x, d, M["norm_f"], c.eps, None, _C._buf(self.dxf, n, H), None, None)
         self._tr("mtp.x_out", x)
@@ -480,8 +496,7 @@ class HybridModel:
         of the verify's token among them), the first `width` become tree rows."""
         c, T = self.cfg, self.tree
         nout = 7 if c.auto else width
-        _C.mtp_prep_draft(self.st, k, self.ftab.view(1, 1, c.cap, c.rotary // 2, 2, 2), self.dfreqs, self.mpos, self.mseq)
-        self.mtp_block(1, tok, h, self.dfreqs.view(1, c.rotary // 2, 2, 2), self.mpos[:1], self.mseq, None)
+        self.mtp_block(1, tok, h, self.dfreqs.view(1, c.rotary // 2, 2, 2), self.mpos[:1], self.mseq, None, depth=k)
         xf = self.dxf[:1]
         picked = None
         if c.head == "int8":
@@ -494,8 +509,7 @@ class HybridModel:
             else:
                 _C.int8_linear_prequantized(qx, sx, self.lm8, self.lm8_s, tiled=True, out=self.dlogits)
         elif c.two_stage:
-            q, s = _C.quant_rows(xf)
-            _C.stream_gemv(q, s.view(-1), [self.lm4], [self.dlogits])
+            _C.stream_gemv(self.dqx[:1], self.dsx[:1], [self.lm4], [self.dlogits])
             _C.draft_pick_bf16(self.dlogits.view(-1), xf.view(-1), self.lm_rows, nout, False, self.dtop[k], None,
                                self.dtok[k], self.vtok.view(-1), T["fill_rows"][k], tiled=False)
             picked = self.dtop[k]

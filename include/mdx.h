@@ -506,6 +506,36 @@ int mdx_attn_exact(const uint16_t* q, int64_t q_head_stride, int64_t q_row_strid
                    const int32_t* mask, uint16_t* out, int64_t H, int64_t Hk, int64_t S, int64_t D, int64_t cap,
                    float scale, void* stream);
 
+/* ---- launches of the MTP draft block that take their elementwise neighbours along ------------- */
+
+/* mdx_attn_decode, its output times a sigmoid: out <- bf16(out * sig_lut[gate]), the gate of (row, head, d) at
+ * gate[row * gate_row_stride + 2 D head + D + d] (mdx_draft_sigmoid_mul's layout and arithmetic). */
+int mdx_attn_decode_gated(const uint16_t* q, int64_t q_head_stride, int64_t q_row_stride, const uint16_t* key,
+                    const uint16_t* value, const int32_t* seqlen, const uint16_t* xk, int64_t xk_head_stride,
+                    int64_t xk_row_stride, const uint16_t* xv, int64_t xv_head_stride, int64_t xv_row_stride,
+                    const int32_t* mask, uint16_t* out, int64_t H,
+                    int64_t Hk, int64_t S, int64_t D, int64_t cap, int64_t chunks_hint,
+                    const uint16_t* gate, int64_t gate_row_stride, const uint16_t* sig_lut, void* workspace,
+                    size_t workspace_bytes, void* stream);
+
+/* out bf16 [rows, I] = bf16(silu_lut[g] * u), g | u = mdx_bf16_linear's outputs over the tile-major weights [2 I, K]
+ * (gate rows, then up rows), the bits of that launch followed by mdx_draft_silu_mul; 1..16 rows, where
+ * mdx_bf16_gate_up_fits(I, K). */
+int32_t mdx_bf16_gate_up_fits(int64_t I, int64_t K);
+int mdx_bf16_gate_up(const uint16_t* x, const uint16_t* w, const uint16_t* silu_lut, uint16_t* out, int64_t rows, int64_t I,
+                     int64_t K, void* stream);
+
+/* x = bf16(x + h) in place (h may be NULL), xn = RMSNorm(x), qx / sx = mdx_rot_quant's quantisation of xn without
+ * rotation (mdx_draft_norm_rot_quant followed by the row prep, in one launch). */
+int mdx_draft_norm_quant(uint16_t* x, const uint16_t* h, const uint16_t* w, float eps, uint16_t* xn, int8_t* qx, float* sx,
+                         int64_t rows, int64_t H, void* stream);
+
+/* mdx_draft_embed_norm_cat of one row gathered from a bf16 table, and mdx_mtp_prep_draft, in one launch. */
+int mdx_draft_embed_prep(const int64_t* token, int64_t V, const uint16_t* emb, const uint16_t* hidden, const uint16_t* we,
+                         const uint16_t* wh, float eps_e, float eps_h, uint16_t* out, int64_t H, const int64_t* st, int64_t k,
+                         const float* ftab, int64_t ftab_rows, int64_t row_elems, float* freqs, int64_t* mpos, int64_t npos,
+                         int32_t* mseq, void* stream);
+
 /* ---- many-row forms for the prompt prefill ---------------------------------------------------
  * The reference has none (its prefill is the host framework's); these carry the decode operators' contracts to any
  * row count, so that a prompt streams each weight once per up to 128 rows. */
