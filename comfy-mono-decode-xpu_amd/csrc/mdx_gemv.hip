@@ -38,6 +38,8 @@
 #include <stdio.h>
 #include <vector>
 #include <stdlib.h>
+#include <string.h>
+#include <unistd.h>
 
 #include "mdx_common.hpp"
 #include "mdx_gdn_ops.hpp"
@@ -1655,11 +1657,22 @@ int setup_gemv(const mdx_w4* const* ws, int nm, bool pair, const int8_t* xq, con
     return MDX_OK;
 }
 
+// A tuning variable of the environment (MDX_*), read at each launch: one pass over the environment tells whether any is set
+// (each getenv walks all of it, and a launch asks for several).
+struct TuneEnv {
+    bool any = false;
+    TuneEnv() {
+        for (char** e = environ; e && *e && !any; ++e) any = (*e)[0] == 'M' && !strncmp(*e, "MDX_", 4);
+    }
+    const char* get(const char* name) const { return any ? getenv(name) : nullptr; }
+};
+
 // The launch geometry: TPW tiles per work-group, KS K-slices per tile (at most 16 waves per
 // work-group): the smallest split that puts >= 3072 waves on the chip (12 per CU), but no slice
 // shorter than 4 chunks, measured best on MI355X for the 8-52 MB matrices of this model (longer
 // streams per wave beat more, shorter waves: 4096 x 4096 takes 6.4 us at 8 slices against 7.6 at 12).
 void gemv_geometry(int total, int K, bool pair, int rows, int& TPW, int& KS) {
+    const TuneEnv tune;
     TPW = pair ? 2 : 1;
     // more than 8 rows: about one work-group per CU (up to six tiles each). Every work-group stages
     // all of its rows' K range, so wider work-groups stage less per CU: the 16-row MLP 46.3 -> 41.3 us
@@ -1684,7 +1697,7 @@ void gemv_geometry(int total, int K, bool pair, int rows, int& TPW, int& KS) {
     }
     // MDX_GEMV_TPW / MDX_GEMV_KS override the geometry (tuning sweeps); MDX_GEMV_PAIR_TPW / _KS only that of
     // gate/up pairs
-    if (const char* env = pair ? getenv("MDX_GEMV_PAIR_TPW") : nullptr) {
+    if (const char* env = pair ? tune.get("MDX_GEMV_PAIR_TPW") : nullptr) {
         const int tpw = atoi(env);
         if (tpw >= 2 && tpw <= 6 && tpw % 2 == 0) TPW = tpw;
         KS = 1;
@@ -1694,15 +1707,15 @@ void gemv_geometry(int total, int K, bool pair, int rows, int& TPW, int& KS) {
             if (int64_t(total) * d >= 3072) break;
         }
     }
-    if (const char* env = pair ? getenv("MDX_GEMV_PAIR_KS") : nullptr) {
+    if (const char* env = pair ? tune.get("MDX_GEMV_PAIR_KS") : nullptr) {
         const int ks = atoi(env);
         if (ks >= 1 && ks * TPW <= 16 && NC % ks == 0) KS = ks;
     }
-    if (const char* env = getenv("MDX_GEMV_TPW")) {
+    if (const char* env = tune.get("MDX_GEMV_TPW")) {
         const int tpw = atoi(env);
         if (tpw >= 1 && tpw <= 6 && (!pair || tpw % 2 == 0)) TPW = tpw;  // the parameter block holds 6 tiles
     }
-    if (const char* env = getenv("MDX_GEMV_KS")) {
+    if (const char* env = tune.get("MDX_GEMV_KS")) {
         const int ks = atoi(env);
         if (ks >= 1 && ks * TPW <= 16 && NC % ks == 0) KS = ks;
     }
@@ -1837,7 +1850,8 @@ int run_gemv(const mdx_w4* const* ws, int nm, bool pair, const int8_t* xq, const
     // tables save; there the lanes build their tables in the loop). Tables select the table-only
     // variants, which run on the MFMA kernel at every row count (at one row too: the products leave
     // the VALU to the decode).
-    const char* te = getenv("MDX_GEMV_TBL");  // MDX_GEMV_TBL=8: the 8-byte tier whenever it applies (tests)
+    const TuneEnv tune;
+    const char* te = tune.get("MDX_GEMV_TBL");  // MDX_GEMV_TBL=8: the 8-byte tier whenever it applies (tests)
     const bool tbl8 = te && atoi(te) == 8 && !a.cb;
     if (xg && a.lgG >= 7) {
         a.tbl = tbl8 ? 2 : 1;  // (without the rows in LDS a work-group's tables always leave room for others)
@@ -1874,7 +1888,7 @@ int run_gemv(const mdx_w4* const* ws, int nm, bool pair, const int8_t* xq, const
     MDX_CHECK(!(mfma && a.xp_x) || a.tbl, "row-prep GEMV geometry (one row takes the VALU kernel or the tables)");
     // per-wave one-shots: one int8 row, caller-asserted integral scales with the default codebook,
     // G128, 16-byte runs of scales per slice and per row (MDX_GEMV_PWO=0 turns them off)
-    const char* pe = getenv("MDX_GEMV_PWO");
+    const char* pe = tune.get("MDX_GEMV_PWO");
     const int NCk = a.K / CHUNK_K;
     a.pwo = !mfma && rows == 1 && a.assume_int && !a.cb && a.lgG == 7 &&
             (NCk / a.KS) * esz % 16 == 0 && (a.K >> 7) * esz % 16 == 0 && aligned(xq, 16) && !(pe && atoi(pe) == 0);

@@ -17,7 +17,7 @@ import weakref
 import torch
 
 from . import _lib
-from .layout import W4, classify_rotation
+from .layout import _SDT, W4, classify_rotation
 
 _OUT_DT = {0: (torch.float32, _lib.DT_F32), 2: (torch.bfloat16, _lib.DT_BF16)}
 
@@ -53,6 +53,11 @@ def _codebook(cb):
 
 
 def _w4(q, s, sc, cb, tiled=False) -> W4:
+    return W4(q, s, sc, _w4_checked(q, s, sc, cb), _lib.LAYOUT_TILE if tiled else _lib.LAYOUT_ROW, _lib.DECODE_AUTO)
+
+
+def _w4_checked(q, s, sc, cb):
+    """The four contract tensors checked; the codebook (None when it is the default one)."""
     _dev(q, "packed W4")
     _check(q.dtype in (torch.int8, torch.uint8) and q.dim() == 2 and q.is_contiguous(),
            "packed must be contiguous int8 [N, K/2]")
@@ -62,29 +67,37 @@ def _w4(q, s, sc, cb, tiled=False) -> W4:
     _check(sc.dtype == torch.float32 and sc.is_contiguous() and sc.numel() == q.shape[0], "s_channel f32 [N]")
     if cb is not None:
         _check(cb.dtype == torch.float32 and cb.numel() == 16 and cb.is_contiguous(), "codebook f32 [16]")
-    return W4(q, s, sc, _codebook(cb), _lib.LAYOUT_TILE if tiled else _lib.LAYOUT_ROW, _lib.DECODE_AUTO)
+    return _codebook(cb)
 
 
 def w4a8_decode_linear(x, x_scale, packed, s_rel, s_channel, codebook=None, residual=None, group_size=16,
                        out_dtype_code=2, cols=0, fast=False):
     """Reference csrc/w4a8_decode.sycl:325-370: one fused small-M W4A8 linear (row-major weights)."""
     _dev(x, "x")
-    _check(x.dtype == torch.int8 and x.dim() == 2 and x.is_contiguous(), "x must be contiguous int8 [M, K]")
+    if not (x.dtype == torch.int8 and x.dim() == 2 and x.is_contiguous()):
+        raise RuntimeError("x must be contiguous int8 [M, K]")
     M, K = x.shape
+    xp = x.data_ptr()
     _check(1 <= M <= 16, "1 <= M <= 16")
-    _check(x.data_ptr() % 16 == 0, "x must be 16-byte aligned")
-    w = _w4(packed, s_rel, s_channel, codebook)
-    _check(w.k == K, "packed must be [N, K/2]")
-    _check(w.group_size == group_size, f"s_rel has {s_rel.shape[1]} groups, not K / group_size")
-    _check(x_scale.dtype == torch.float32 and x_scale.is_contiguous() and x_scale.numel() == M, "x_scale f32 [M]")
+    _check(xp % 16 == 0, "x must be 16-byte aligned")
+    cb = _w4_checked(packed, s_rel, s_channel, codebook)
+    N, K2 = packed.shape
+    groups = s_rel.shape[1]
+    _check(2 * K2 == K, "packed must be [N, K/2]")
+    if K // groups != group_size:
+        raise RuntimeError(f"s_rel has {groups} groups, not K / group_size")
+    if not (x_scale.dtype == torch.float32 and x_scale.is_contiguous() and x_scale.numel() == M):
+        raise RuntimeError("x_scale f32 [M]")
     _check(out_dtype_code in _OUT_DT, "out dtype fp32 or bf16")
     dt, code = _OUT_DT[out_dtype_code]
-    out = torch.empty(M, w.n, dtype=dt, device=x.device)
+    out = torch.empty((M, N), dtype=dt, device=x.device)
     if residual is not None:
-        _check(residual.dtype == dt and residual.is_contiguous() and residual.numel() == M * w.n,
+        _check(residual.dtype == dt and residual.is_contiguous() and residual.numel() == M * N,
                "residual must match output")
-    _lib.call("mdx_w4a8_decode_linear", _lib.ptr(x), _lib.ptr(x_scale), w.struct(), _lib.ptr(residual), _lib.ptr(out),
-              code, M, _lib.stream_of(x))
+    w = _lib.MdxW4(packed.data_ptr(), s_rel.data_ptr(), s_channel.data_ptr(), None if cb is None else cb.data_ptr(), N, K,
+                   K // groups, _SDT[s_rel.dtype], _lib.LAYOUT_ROW, _lib.DECODE_AUTO, 0)
+    _lib.call("mdx_w4a8_decode_linear", xp, x_scale.data_ptr(), w, _lib.ptr(residual), out.data_ptr(), code, M,
+              _lib.stream_of(x))
     return out
 
 

@@ -118,13 +118,9 @@ class W4:
 
     def struct(self):
         if self._struct is None:
-            st = _lib.MdxW4()
-            st.q, st.s_rel = self.q.data_ptr(), self.s.data_ptr()
-            st.s_channel = self.sc.data_ptr()
-            st.codebook = None if self.cb is None else self.cb.data_ptr()
-            st.n, st.k, st.group_size = self.n, self.k, self.group_size
-            st.s_dtype = _SDT[self.s.dtype]
-            st.layout, st.decode = self.layout, self.decode
+            q, sr, k = self.q, self.s, self.q.shape[1] * 2
+            st = _lib.MdxW4(q.data_ptr(), sr.data_ptr(), self.sc.data_ptr(), None if self.cb is None else self.cb.data_ptr(),
+                            q.shape[0], k, k // sr.shape[1], _SDT[sr.dtype], self.layout, self.decode, 0)
             self._struct = st
         return self._struct
 
