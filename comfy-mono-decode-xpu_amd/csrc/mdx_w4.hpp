@@ -26,11 +26,38 @@ __device__ __forceinline__ Lut make_lut(float s, const float* cb) {
     return L;
 }
 
+// The default codebook's 16-byte table from its magnitudes (make_lut_c8's bytes): byte reversal and
+// a carry-free negation of four int8 at once (~b + 1 per byte; no byte is -128 after the clamp).
+__device__ __forceinline__ Lut lut_from_q8(uint32_t qa, uint32_t qb) {
+    auto neg4 = [](uint32_t b) {
+        const uint32_t n = ~b;
+        return ((n & 0x7F7F7F7Fu) + 0x01010101u) ^ (n & 0x80808080u);
+    };
+    Lut L;
+    L.w[0] = neg4(__builtin_amdgcn_perm(0u, qb, 0x00010203u));  // -q8, -q7, -q6, -q5
+    L.w[1] = neg4(__builtin_amdgcn_perm(0u, qa, 0x00010203u));  // -q4 .. -q1
+    L.w[2] = __builtin_amdgcn_perm(0u, qa, 0x0201000Cu);        // 0, q1, q2, q3
+    L.w[3] = __builtin_amdgcn_perm(qb, qa, 0x06050403u);        // q4 .. q7
+    return L;
+}
+
 // The table of the default codebook (c - 8) from its eight magnitudes: rint and the clamp are odd
 // functions and (-k) s = -(k s) exactly, so entry 8 - k is the negation of q(k s) = clamp(rint(k s),
 // +-127) (NaN -> 0) and entry 8 is 0 (0 * s rounds to 0, or is NaN -> 0): eight products instead of
 // sixteen, the same bytes as make_lut.
 __device__ __forceinline__ Lut make_lut_c8(float s) {
+    if (__builtin_amdgcn_ballot_w64(!(fabsf(s) <= 15.875f)) == 0) {
+        // every |k s| of the active lanes at most 127 (no NaN): fl32(k s) + 1.5 2^23 rounds to an integer once more, to
+        // nearest even as rint does, and holds it in its low byte: two instructions per magnitude and no clamp (the tables
+        // that lanes build per chunk: f32 scales per 32, 8 rows, 12288 x 4096 15.0 -> 13.2 us, 4096 x 12288 15.5 -> 13.8)
+        uint32_t u[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) u[k] = __float_as_uint(__fadd_rn(__fmul_rn(float(k + 1), s), 12582912.f));
+        auto four = [](uint32_t b0, uint32_t b1, uint32_t b2, uint32_t b3) {
+            return __builtin_amdgcn_perm(__builtin_amdgcn_perm(b3, b2, 0x0C0C0400u), __builtin_amdgcn_perm(b1, b0, 0x0C0C0400u), 0x05040100u);
+        };
+        return lut_from_q8(four(u[0], u[1], u[2], u[3]), four(u[4], u[5], u[6], u[7]));
+    }
     int q[9];
     q[0] = 0;
 #pragma unroll
@@ -78,21 +105,6 @@ __device__ __forceinline__ uint2 make_q8_f16(uint32_t sbits) {
         r[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(kk, s2, magic));
     }
     return make_uint2(__builtin_amdgcn_perm(r[1], r[0], 0x06040200u), __builtin_amdgcn_perm(r[3], r[2], 0x06040200u));
-}
-
-// The default codebook's 16-byte table from its magnitudes (make_lut_c8's bytes): byte reversal and
-// a carry-free negation of four int8 at once (~b + 1 per byte; no byte is -128 after the clamp).
-__device__ __forceinline__ Lut lut_from_q8(uint32_t qa, uint32_t qb) {
-    auto neg4 = [](uint32_t b) {
-        const uint32_t n = ~b;
-        return ((n & 0x7F7F7F7Fu) + 0x01010101u) ^ (n & 0x80808080u);
-    };
-    Lut L;
-    L.w[0] = neg4(__builtin_amdgcn_perm(0u, qb, 0x00010203u));  // -q8, -q7, -q6, -q5
-    L.w[1] = neg4(__builtin_amdgcn_perm(0u, qa, 0x00010203u));  // -q4 .. -q1
-    L.w[2] = __builtin_amdgcn_perm(0u, qa, 0x0201000Cu);        // 0, q1, q2, q3
-    L.w[3] = __builtin_amdgcn_perm(qb, qa, 0x06050403u);        // q4 .. q7
-    return L;
 }
 
 // four codes (one per byte, values 0..15) -> four int8 via the 16-byte table
