@@ -612,10 +612,19 @@ __global__ __launch_bounds__(MERGE_T) void attn_merge_kernel(AttnArgs a) {
     const int i0 = min(lane, max(np - 1, 0)), i1 = min(lane + 64, max(np - 1, 0));
     float m0 = base[slot(i0) * (32 + 16 * D) + row], m1 = base[slot(i1) * (32 + 16 * D) + row];
     const float l0 = base[slot(i0) * (32 + 16 * D) + 16 + row], l1 = base[slot(i1) * (32 + 16 * D) + 16 + row];
+    // (few partials of a small head: a third of the loads; at head_dim 256 the branch costs more than it saves)
     f32x4 ov[PER];
+    auto load_o = [&](auto n) {
 #pragma unroll
-    for (int j = 0; j < PER; ++j)
-        ov[j] = *reinterpret_cast<const f32x4*>(base + slot(min(gi + G * j, max(np - 1, 0))) * (32 + 16 * D) + 32 + row * D + d4);
+        for (int j = 0; j < decltype(n)::value; ++j)
+            ov[j] = *reinterpret_cast<const f32x4*>(base + slot(min(gi + G * j, max(np - 1, 0))) * (32 + 16 * D) + 32 + row * D + d4);
+    };
+    constexpr int FEW = D == 256 ? PER : (PER + 2) / 3;
+    const bool few = np <= FEW * G;  // (uniform)
+#pragma unroll
+    for (int j = FEW; j < PER; ++j) ov[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (few) load_o(std::integral_constant<int, FEW>{});
+    else load_o(std::integral_constant<int, PER>{});
     m0 = lane < np ? m0 : -INFINITY;
     m1 = lane + 64 < np ? m1 : -INFINITY;
     auto ror = [](float v, auto ctl) {
