@@ -20,7 +20,8 @@
 // replays for any context length.
 //
 // One work-group per (kv head, chunk) over all of the kv head's row tiles, K/V read once from HBM into an LDS ring (see
-// the layout note at stage_k). Head_dim 256 (4 kv heads, 8 rows of 4 heads, ctx 8192): 13.7 us per launch; with K rows
+// the layout note at stage_k). Head_dim 256 (4 kv heads, 8 rows of 4 heads, ctx 8192): 14.3 us per launch (13.7 without
+// the maximum per stage, see add_pv); with K rows
 // straight from HBM as MFMA operands, V transposed through LDS and a work-group per (row tile, chunk) it took 23.9 us.
 //
 // The tree-verify form with the Q/K prep (attn2_kernel<.., PREP>, head_dim 128): the launch also does the
@@ -188,6 +189,38 @@ __device__ __forceinline__ void stage_v(u32x2 (&va)[D / 16], u32x2 (&vb)[D / 16]
     }
 }
 
+// O^T += V^T P of one stage: O^T times alpha, the stage's products times beta (OWN only; 1 otherwise).
+// OWN: P is rounded to bf16 against its own stage's maximum, and the products of the 32 tokens are brought to the
+// running maximum in fp32. The weight at the maximum a P is taken against is exactly 1, every other carries bf16's
+// rounding, so the error grows with the tokens per maximum: against one running maximum over a part the outputs lay up to
+// 2 % further from float64 (head_dim 256, ctx 16000: 1.760e-3, with a maximum per 32 tokens 1.709e-3).
+template <int DT, bool OWN>
+__device__ __forceinline__ void add_pv(f32x4 (&acc)[DT], const u32x2 (&va)[DT], const u32x2 (&vb)[DT], const u32x4 pf,
+                                       const float alpha, const float beta) {
+    auto pv = [&](int dt, f32x4 c) {
+        const u32x4 vf = {va[dt].x, va[dt].y, vb[dt].x, vb[dt].y};
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf), c, 0, 0, 0);
+    };
+    // (uniform) some row's maximum is not this stage's: the products go through registers of their own
+    if (OWN && __builtin_amdgcn_ballot_w64(beta != 1.f) != 0) {
+        f32x4 o[DT];
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = pv(dt, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[dt][i] = fmaf(o[dt][i], beta, acc[dt][i] * alpha);
+        return;
+    }
+    // O^T is rescaled only when some row's maximum moved (x * 1 == x: skipping changes no bit)
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) acc[dt] = pv(dt, acc[dt]);
+}
+
 // chunk length (tokens, a multiple of 32 P) and active chunk count for context L over C chunks
 __device__ __forceinline__ void split2(int L, int C, int P, int& T, int& active) {
     const int per = (L + C - 1) / C, q = A2_STEP * P;
@@ -207,6 +240,8 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
     // barrier per stage): filled one stage ahead, the second stage's load would go out only after the first had landed.
     // Longer rings fill NS - 1 ahead and refill the slot of the stage before at the top of a stage.
     constexpr bool WHOLE = NS == 2;
+    // head_dim 256's parts are up to 96 tokens and more long (two parts per chunk): a maximum per stage (add_pv)
+    constexpr bool OWN = D == 256;
     constexpr int AHEAD = WHOLE ? NS : NS - 1;  // stages issued by the prologue
     static_assert(NS >= 2 && PER >= 1 && (AHEAD - 1) * 2 * PER <= 63, "ring geometry");
     extern __shared__ __align__(16) unsigned char smem[];
@@ -498,33 +533,27 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
         // a row with nothing admitted yet subtracts 0, so -inf - -inf never forms
         const float msub = mnew == -INFINITY ? 0.f : mnew;
         const float alpha = __builtin_amdgcn_exp2f(m - msub);
+        // the maximum that P is taken against, and the factor from it to the running one (OWN: see below)
+        const float pmax = !OWN ? msub : (mx == -INFINITY ? 0.f : mx);
+        const float beta = !OWN ? 1.f : __builtin_amdgcn_exp2f(mx - msub);
         float p[2][4], ps = 0.f;
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
             for (int i = 0; i < 4; i += 2) {
-                p[tt][i] = __builtin_amdgcn_exp2f(z[tt][i] - msub);
-                p[tt][i + 1] = __builtin_amdgcn_exp2f(z[tt][i + 1] - msub);
+                p[tt][i] = __builtin_amdgcn_exp2f(z[tt][i] - pmax);
+                p[tt][i + 1] = __builtin_amdgcn_exp2f(z[tt][i + 1] - pmax);
                 bfround2(p[tt][i], p[tt][i + 1]);
                 ps += p[tt][i];
                 ps += p[tt][i + 1];
             }
         ps = sum_x32(sum_x16(ps));
-        l = l * alpha + ps;
+        l = l * alpha + (OWN ? ps * beta : ps);
         m = mnew;
-        // O^T is rescaled only when some row's maximum moved (x * 1 == x: skipping changes no bit)
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
-        }
         // p holds bf16 values: their top halves are the MFMA operand
         auto top2 = [](float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); };
         const u32x4 pf = {top2(p[0][0], p[0][1]), top2(p[0][2], p[0][3]), top2(p[1][0], p[1][1]), top2(p[1][2], p[1][3])};
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            const u32x4 vf = {va[dt].x, va[dt].y, vb2[dt].x, vb2[dt].y};
-            acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf), acc[dt], 0, 0, 0);
-        }
+        add_pv<DT, OWN>(acc, va, vb2, pf, alpha, beta);
     }
 
     // the work-group's partial per row tile: (m, l, O) of its rows; P parts merge through LDS first
