@@ -20,8 +20,8 @@
 // replays for any context length.
 //
 // One work-group per (kv head, chunk) over all of the kv head's row tiles, K/V read once from HBM into an LDS ring (see
-// the layout note at stage_k). Head_dim 256 (4 kv heads, 8 rows of 4 heads, ctx 8192): 14.3 us per launch (13.7 without
-// the maximum per stage, see add_pv); with K rows
+// the layout note at stage_k). Head_dim 256 (4 kv heads, 8 rows of 4 heads, ctx 8192): 14.0 us per launch (13.7 without
+// the maximum per stage, add_own_max); with K rows
 // straight from HBM as MFMA operands, V transposed through LDS and a work-group per (row tile, chunk) it took 23.9 us.
 //
 // The tree-verify form with the Q/K prep (attn2_kernel<.., PREP>, head_dim 128): the launch also does the
@@ -189,36 +189,28 @@ __device__ __forceinline__ void stage_v(u32x2 (&va)[D / 16], u32x2 (&vb)[D / 16]
     }
 }
 
-// O^T += V^T P of one stage: O^T times alpha, the stage's products times beta (OWN only; 1 otherwise).
-// OWN: P is rounded to bf16 against its own stage's maximum, and the products of the 32 tokens are brought to the
-// running maximum in fp32. The weight at the maximum a P is taken against is exactly 1, every other carries bf16's
-// rounding, so the error grows with the tokens per maximum: against one running maximum over a part the outputs lay up to
-// 2 % further from float64 (head_dim 256, ctx 16000: 1.760e-3, with a maximum per 32 tokens 1.709e-3).
-template <int DT, bool OWN>
-__device__ __forceinline__ void add_pv(f32x4 (&acc)[DT], const u32x2 (&va)[DT], const u32x2 (&vb)[DT], const u32x4 pf,
-                                       const float alpha, const float beta) {
-    auto pv = [&](int dt, f32x4 c) {
+// The MFMA operand of P^T: bf16 values in fp32, their top halves.
+__device__ __forceinline__ u32x4 p_operand(const float (&p)[2][4]) {
+    auto top2 = [](float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); };
+    return u32x4{top2(p[0][0], p[0][1]), top2(p[0][2], p[0][3]), top2(p[1][0], p[1][1]), top2(p[1][2], p[1][3])};
+}
+
+// O^T = alpha O^T + beta V^T P of a stage whose P was rounded to bf16 against its own maximum: its products are brought
+// to the running maximum in fp32. The weight at the maximum that P is taken against is exactly 1, every other carries
+// bf16's rounding, so the error grows with the tokens per maximum: against one running maximum over a part the outputs
+// lay up to 2 % further from float64 (head_dim 256, ctx 16000: 1.760e-3, with a maximum per 32 tokens 1.709e-3), against
+// one over the whole prefix in the prefill form up to 8 % further than the same rows in chains of 16 (500 rows after 500,
+// head_dim 128: 1.862e-3, per stage 1.722e-3 like the chains).
+template <int DT>
+__device__ __forceinline__ void add_own_max(f32x4 (&acc)[DT], const u32x2 (&va)[DT], const u32x2 (&vb)[DT], const u32x4 pf,
+                                            const float alpha, const float beta) {
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
         const u32x4 vf = {va[dt].x, va[dt].y, vb[dt].x, vb[dt].y};
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf), c, 0, 0, 0);
-    };
-    // (uniform) some row's maximum is not this stage's: the products go through registers of their own
-    if (OWN && __builtin_amdgcn_ballot_w64(beta != 1.f) != 0) {
-        f32x4 o[DT];
+        const f32x4 o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf), f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) o[dt] = pv(dt, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[dt][i] = fmaf(o[dt][i], beta, acc[dt][i] * alpha);
-        return;
+        for (int i = 0; i < 4; ++i) acc[dt][i] = fmaf(o[i], beta, acc[dt][i] * alpha);
     }
-    // O^T is rescaled only when some row's maximum moved (x * 1 == x: skipping changes no bit)
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
-    }
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt] = pv(dt, acc[dt]);
 }
 
 // chunk length (tokens, a multiple of 32 P) and active chunk count for context L over C chunks
@@ -240,7 +232,7 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
     // barrier per stage): filled one stage ahead, the second stage's load would go out only after the first had landed.
     // Longer rings fill NS - 1 ahead and refill the slot of the stage before at the top of a stage.
     constexpr bool WHOLE = NS == 2;
-    // head_dim 256's parts are up to 96 tokens and more long (two parts per chunk): a maximum per stage (add_pv)
+    // head_dim 256's parts are up to 96 tokens and more long (two parts per chunk): a maximum per stage (add_own_max)
     constexpr bool OWN = D == 256;
     constexpr int AHEAD = WHOLE ? NS : NS - 1;  // stages issued by the prologue
     static_assert(NS >= 2 && PER >= 1 && (AHEAD - 1) * 2 * PER <= 63, "ring geometry");
@@ -533,7 +525,7 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
         // a row with nothing admitted yet subtracts 0, so -inf - -inf never forms
         const float msub = mnew == -INFINITY ? 0.f : mnew;
         const float alpha = __builtin_amdgcn_exp2f(m - msub);
-        // the maximum that P is taken against, and the factor from it to the running one (OWN: see below)
+        // the maximum that P is taken against, and the factor from it to the running one (OWN: add_own_max)
         const float pmax = !OWN ? msub : (mx == -INFINITY ? 0.f : mx);
         const float beta = !OWN ? 1.f : __builtin_amdgcn_exp2f(mx - msub);
         float p[2][4], ps = 0.f;
@@ -550,10 +542,21 @@ __global__ __launch_bounds__(64 * NWV) void attn2_kernel(AttnArgs a) {
         ps = sum_x32(sum_x16(ps));
         l = l * alpha + (OWN ? ps * beta : ps);
         m = mnew;
-        // p holds bf16 values: their top halves are the MFMA operand
-        auto top2 = [](float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); };
-        const u32x4 pf = {top2(p[0][0], p[0][1]), top2(p[0][2], p[0][3]), top2(p[1][0], p[1][1]), top2(p[1][2], p[1][3])};
-        add_pv<DT, OWN>(acc, va, vb2, pf, alpha, beta);
+        if constexpr (OWN) {
+            add_own_max<DT>(acc, va, vb2, p_operand(p), alpha, beta);
+        } else {
+            // O^T is rescaled only when some row's maximum moved (x * 1 == x: skipping changes no bit)
+            if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
+            }
+            const u32x4 pf = p_operand(p);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                const u32x4 vf = {va[dt].x, va[dt].y, vb2[dt].x, vb2[dt].y};
+                acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf), acc[dt], 0, 0, 0);
+            }
+        }
     }
 
     // the work-group's partial per row tile: (m, l, O) of its rows; P parts merge through LDS first
@@ -777,52 +780,39 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
         u32x2 va[DT], vb2[DT];
         stage_v<D>(va, vb2, lds_addr(kd + STAGE) + (4 * g + (c16 >> 2)) * 32 + (c16 & 3) * 8);
         const int nvalid = L + row + 1 - t0;  // this row's tokens of the stage
-        float z[2][4], mx = -INFINITY;
-        if (__builtin_amdgcn_ballot_w64(nvalid < A2_STEP) == 0) {
+        // a stage whole for every row takes its 32 tokens at once; one on the diagonal as two halves with a maximum each,
+        // as a chain of 16 rows takes its own rows apart from the prefix (add_own_max)
+        const int parts = __builtin_amdgcn_ballot_w64(nvalid < A2_STEP) == 0 ? 1 : 2;  // (uniform in the wave)
+        for (int part = 0; part < parts; ++part) {
+            float z[2][4], mx = -INFINITY;
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    z[tt][i] = st[tt][i] * a.zscale;
+                    const bool in = parts == 1 || (tt == part && 16 * tt + 4 * g + i < nvalid);
+                    z[tt][i] = in ? st[tt][i] * a.zscale : -INFINITY;
                     mx = fmaxf(mx, z[tt][i]);
                 }
-        } else {
+            mx = max_x32(max_x16(mx));
+            const float mnew = fmaxf(m, mx);
+            const float msub = mnew == -INFINITY ? 0.f : mnew;
+            const float alpha = __builtin_amdgcn_exp2f(m - msub);
+            const float pmax = mx == -INFINITY ? 0.f : mx, beta = __builtin_amdgcn_exp2f(mx - msub);
+            float p[2][4], ps = 0.f;
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    z[tt][i] = 16 * tt + 4 * g + i < nvalid ? st[tt][i] * a.zscale : -INFINITY;
-                    mx = fmaxf(mx, z[tt][i]);
+                for (int i = 0; i < 4; i += 2) {
+                    p[tt][i] = __builtin_amdgcn_exp2f(z[tt][i] - pmax);
+                    p[tt][i + 1] = __builtin_amdgcn_exp2f(z[tt][i + 1] - pmax);
+                    bfround2(p[tt][i], p[tt][i + 1]);
+                    ps += p[tt][i];
+                    ps += p[tt][i + 1];
                 }
-        }
-        mx = max_x32(max_x16(mx));
-        const float mnew = fmaxf(m, mx);
-        const float msub = mnew == -INFINITY ? 0.f : mnew;
-        const float alpha = __builtin_amdgcn_exp2f(m - msub);
-        float p[2][4], ps = 0.f;
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int i = 0; i < 4; i += 2) {
-                p[tt][i] = __builtin_amdgcn_exp2f(z[tt][i] - msub);
-                p[tt][i + 1] = __builtin_amdgcn_exp2f(z[tt][i + 1] - msub);
-                bfround2(p[tt][i], p[tt][i + 1]);
-                ps += p[tt][i];
-                ps += p[tt][i + 1];
-            }
-        ps = sum_x32(sum_x16(ps));
-        l = l * alpha + ps;
-        m = mnew;
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
-        }
-        auto top2 = [](float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); };
-        const u32x4 pf = {top2(p[0][0], p[0][1]), top2(p[0][2], p[0][3]), top2(p[1][0], p[1][1]), top2(p[1][2], p[1][3])};
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            const u32x4 vf = {va[dt].x, va[dt].y, vb2[dt].x, vb2[dt].y};
-            acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf), acc[dt], 0, 0, 0);
+            ps = sum_x32(sum_x16(ps));
+            l = l * alpha + ps * beta;
+            m = mnew;
+            add_own_max<DT>(acc, va, vb2, p_operand(p), alpha, beta);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into this work-group's LDS may outlive it

@@ -55,3 +55,39 @@ def test_decode_attention_head_dim_256(C, dev, H, Hk, S, L):
         v[:L], v[L + pad:] = val[0, kh, :L].double(), xv[0, kh].double()
         heads.append((out[:, kh * gr:(kh + 1) * gr].transpose(0, 1).reshape(-1, D), z, v))
     _no_further_than_blocks(heads, f"H={H} Hk={Hk} S={S} L={L}")
+
+
+@pytest.mark.parametrize("H,Hk,D,L,S", [(32, 8, 128, 0, 1000), (32, 8, 128, 500, 500), (16, 8, 64, 0, 200), (8, 2, 64, 1000, 300)])
+def test_prefill_attention(C, dev, H, Hk, D, L, S):
+    """Also no further than the same rows in chains of 16 through the decode attention."""
+    from mdx import _lib
+    gr, cap = H // Hk, L + S + 16
+    g = torch.Generator(device=dev).manual_seed(L + S)
+    r = lambda *s: torch.randn(*s, generator=g, device=dev).bfloat16()  # noqa: E731
+    q = (torch.randn(1, H, S, D, generator=g, device=dev) * 2).bfloat16()
+    k, v = r(1, Hk, cap, D), r(1, Hk, cap, D)
+    out = torch.empty(S, H * D, dtype=torch.bfloat16, device=dev)
+    seq = torch.tensor([L], dtype=torch.int32, device=dev)
+    _lib.call("mdx_attn_prefill", _lib.ptr(q), S * D, D, _lib.ptr(k), _lib.ptr(v), _lib.ptr(seq), _lib.ptr(out), H, Hk, S,
+              D, cap, _lib.stream_of(q))
+    chains = torch.empty_like(out)
+    for s0 in range(0, S, 16):
+        n = min(16, S - s0)
+        new = slice(L + s0, L + s0 + n)
+        mask = torch.tensor([(1 << (i + 1)) - 1 for i in range(n)], dtype=torch.int32, device=dev)
+        chains[s0:s0 + n] = C.attn_dpas(q[:, :, s0:s0 + n], k, v, torch.tensor([L + s0], dtype=torch.int32, device=dev),
+                                        k[:, :, new], v[:, :, new], mask).view(n, -1)
+    allow = (torch.arange(L + S, device=dev)[None] <= L + torch.arange(S, device=dev)[:, None]).repeat(gr, 1)
+    heads, errs = [], [0.0, 0.0]
+    out, chains = (t.double().view(S, H, D) for t in (out, chains))
+    for kh in range(Hk):
+        own = slice(kh * gr, (kh + 1) * gr)
+        z = q[0, own].double().reshape(-1, D) @ k[0, kh, :L + S].double().t().contiguous() / math.sqrt(D)
+        z = z.masked_fill(~allow, -math.inf)
+        vv = v[0, kh, :L + S].double()
+        want = _softmax(z, vv, False)
+        rows = [t[:, own].transpose(0, 1).reshape(-1, D) for t in (out, chains)]
+        errs = [e + float((t - want).norm()) ** 2 for e, t in zip(errs, rows)]
+        heads.append((rows[0], z, vv))
+    _no_further_than_blocks(heads, f"H={H} Hk={Hk} D={D} L={L} S={S}")
+    assert errs[0] <= errs[1] * 1.003 ** 2, (errs[0] ** 0.5, errs[1] ** 0.5)
