@@ -672,7 +672,8 @@ __global__ __launch_bounds__(MERGE_T) void attn_merge_kernel(AttnArgs a) {
     M = fmaxf(M, ror(M, R2{}));
     M = fmaxf(M, ror(M, R1{}));
     const float w0 = m0 == -INFINITY ? 0.f : exp2f(m0 - M), w1 = m1 == -INFINITY ? 0.f : exp2f(m1 - M);
-    float s = (w0 == 0.f ? 0.f : l0 * w0) + (w1 == 0.f ? 0.f : l1 * w1);
+    // (a partial of weight 0 still counts: its NaN, or the infinity of its values, must reach the row)
+    float s = (lane < np ? l0 * w0 : 0.f) + (lane + 64 < np ? l1 * w1 : 0.f);
     s = sum_x32(sum_x16(s));
     s += ror(s, R8{});
     s += ror(s, R4{});
@@ -687,7 +688,7 @@ __global__ __launch_bounds__(MERGE_T) void attn_merge_kernel(AttnArgs a) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
         const float w = wgt[gi + G * j];
-        if (w != 0.f) o += ov[j] * w;  // (an unused record may hold anything)
+        if (gi + G * j < np) o += ov[j] * w;  // (an unused record may hold anything)
     }
     *reinterpret_cast<f32x4*>(&osum[gi][d4]) = o;
     __syncthreads();
