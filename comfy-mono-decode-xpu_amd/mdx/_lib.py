@@ -212,9 +212,17 @@ def gemv_trace():
 
 
 # Arguments go as plain ints (the declared argument types make them pointers): no ctypes object per argument, and the
-# current stream's handle without a torch.cuda.Stream object (1.9 us of an 11 us eager call).
+# current stream's handle without a torch.cuda.Stream object (1.9 us of an 11 us eager call) where this torch has the call.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor):
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    """The handle of the current stream of t's device. A tensor that is not on a ROCm device is refused (its device index,
+    -1, would name the current device, and the launch would take its host pointer)."""
+    d = t.get_device()
+    if d < 0:
+        raise MdxError(f"expected a tensor on the ROCm device, got one on {t.device}")
+    return torch.cuda.current_stream(d).cuda_stream if _raw_stream is None else _raw_stream(d)
 
 
 def ptr(t):
