@@ -38,6 +38,15 @@ struct RunArgs {
     int commit, tail_parity; // rows whose state is kept (the rest: the tail), the tail's buffers
 };
 
+// The control words that a launch takes (uniform in the wave, by every lane's loads): the pending rows' count and parity,
+// and each pending row's slot. One rule for the three kernels, so that invalid words leave every output alone.
+__device__ __forceinline__ bool run_ctl_ok(const RunArgs& a) {
+    const int pending = a.ctl[0], lane = threadIdx.x & 63;
+    if (!gdn_ctl_ok(pending, a.ctl[1], a.slots)) return false;
+    const int sl = lane < pending ? a.ctl[2 + lane] : 0;
+    return __builtin_amdgcn_ballot_w64(sl < 0 || sl >= a.slots) == 0;
+}
+
 constexpr int CR = 16;  // rows per conv work-group (their taps reach 3 rows back)
 constexpr int GR = 16;  // rows per gate wave
 
@@ -45,10 +54,10 @@ constexpr int GR = 16;  // rows per gate wave
 // the gates of one head for GR rows, the head's a / b weights held in registers (gdn_gate_row's sums in its order).
 __global__ __launch_bounds__(256) void gdn_run_prep_kernel(RunArgs a) {
     const int t = threadIdx.x;
+    if (!run_ctl_ok(a)) return;  // (uniform)
     if (int(blockIdx.x) < a.nconv) {
         const int cb = a.C / 512, c = (blockIdx.x % cb) * 512 + 2 * t, r0 = (blockIdx.x / cb) * CR;
         const int pending = a.ctl[0], p = a.ctl[1], S = a.slots;
-        if (!gdn_ctl_ok(pending, p, S)) return;  // (uniform)
         auto row = [&](int r) { return *reinterpret_cast<const uint32_t*>(a.proj + size_t(r) * a.C + c); };
         uint32_t tap[CW];  // the rows before r0, oldest first
         if (r0 == 0) {
@@ -56,8 +65,7 @@ __global__ __launch_bounds__(256) void gdn_run_prep_kernel(RunArgs a) {
 #pragma unroll
             for (int i = 0; i < CW; ++i) {
                 const int j = pending + i;
-                int slot = a.ctl[2 + (j < CW ? 0 : j - CW)];
-                slot = slot < 0 ? 0 : (slot >= S ? S - 1 : slot);
+                const int slot = a.ctl[2 + (j < CW ? 0 : j - CW)];
                 if (j < CW)
                     tap[i] = uint32_t(a.conv_state[c * CW + j]) | (uint32_t(a.conv_state[(c + 1) * CW + j]) << 16);
                 else
@@ -156,10 +164,7 @@ __global__ __launch_bounds__(256) void gdn_run_delta_kernel(RunArgs a) {
     const int t = threadIdx.x, lane = t & 63, h = blockIdx.x / (DH / SC), cs = blockIdx.x % (DH / SC);
     const int S = a.slots, KD = a.HK * DH, kh = h / (a.HV / a.HK);
     const int pending = a.ctl[0], p = a.ctl[1];
-    if (!gdn_ctl_ok(pending, p, S)) return;  // (uniform)
-    // the pending rows are replayed when all their slots are valid
-    const int sl = lane < pending ? a.ctl[2 + lane] : 0;
-    if (__builtin_amdgcn_ballot_w64(sl < 0 || sl >= S) != 0) return;  // (uniform: the decode core leaves the state, too)
+    if (!run_ctl_ok(a)) return;  // (uniform)
     const int col = (t >> 6) * 4 + (lane & 3), rg = lane >> 2;
     float st[RG];
     float* rs = a.rec + (size_t(h) * DH + rg * RG) * DH + cs * SC + col;
@@ -287,8 +292,7 @@ __global__ __launch_bounds__(256) void gdn_run_delta_kernel(RunArgs a) {
 // own: the delta rule's replay may still read the same parity).
 __global__ __launch_bounds__(256) void gdn_run_tail_kernel(RunArgs a) {
     const int tail = a.M - a.commit, S = a.slots, p = a.tail_parity;
-    const int pending = a.ctl[0];
-    if (!gdn_ctl_ok(pending, a.ctl[1], S)) return;  // (uniform)
+    if (!run_ctl_ok(a)) return;  // (uniform)
     const int ng = a.HV * 2, per = a.C / 8;
     for (int i = blockIdx.x * 256 + threadIdx.x; i < S * per; i += gridDim.x * 256) {
         const int r = i / per, c = (i % per) * 8;

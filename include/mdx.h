@@ -576,8 +576,9 @@ int mdx_attn_prefill(const uint16_t* q, int64_t q_head_stride, int64_t q_row_str
  * accepted slots; buffers of the other parity as in mdx_gdn_core), each row's conv output (qkv bf16 [rows, C]), gates
  * (f32 [rows, HV, 2]) and raw delta-rule output (core bf16 [rows, HV * 128]). rec_state and conv_state are left after
  * row rows - tail (at least 3 rows); the last `tail` (0..slots) rows are left pending in the buffers of tail_parity, zeros
- * past them, as a step of those rows leaves them. Invalid control words write nothing. The caller sets ctl for the next
- * step (tail pending rows; 0: none). */
+ * past them, as a step of those rows leaves them. Invalid control words (pending outside 0..slots, parity not 0 / 1, a pending
+ * row's slot outside 0..slots - 1) write nothing: outputs, states and buffers stay as they are. The caller sets ctl for
+ * the next step (tail pending rows; 0: none). */
 int mdx_gdn_run(const uint16_t* proj, const uint16_t* xn, const uint16_t* wa, const uint16_t* wb, int64_t K,
                 const uint16_t* conv_w, uint16_t* conv_state, uint16_t* proj_buf, uint16_t* qkv_buf, float* gates_buf,
                 const int32_t* ctl, const float* dt_bias, const float* g_decay, float* rec_state, float qscale,
