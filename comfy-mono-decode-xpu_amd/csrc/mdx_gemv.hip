@@ -1753,14 +1753,38 @@ bool gemv_gn_fits(const mdx_w4* w, int rows) {
            int64_t(rows) * (w->k / 128) <= int64_t(2) * GN_PASSES * TPW * KS;
 }
 
-// Whether a GEMV of `rows` int8 rows takes them from L2 (SRC_XG): the table variants, where the rows would not fit LDS
-// (128 KiB; they ran in two halves, each streaming the weights: 13 rows, 12288 -> 4096 9.6 + 9.6 -> 10.8 us) and the
-// tables of a work-group's tiles do (16-byte ones: at most 96 KiB). Where the rows fit, LDS is faster: its work-groups
-// share what every wave loads from L2 here (13 rows, gate/up 2 x 12288 x 4096: 14.8 against 17.0 us).
-bool xg_fits(const mdx_w4& w, int rows, bool other_src) {
-    if (rows <= 8 || int64_t(rows) * w.k <= 128 * 1024 || other_src || w.group_size < 16) return false;
-    if (w.s_dtype == MDX_DT_FP8E4M3 && w.group_size < 128) return w.k / w.group_size <= 2048;
-    return w.decode != MDX_DECODE_INTEGRAL && w.group_size >= 128 && w.k / w.group_size <= 192;
+constexpr size_t LDS_MAX = 160 * 1024;
+
+// Whether a GEMV of `rows` int8 rows takes them from L2 (SRC_XG), and through which tables (0: it does not). The table
+// variants do, where the rows would not fit LDS (128 KiB; they ran in two halves, each streaming the weights: 13 rows,
+// 12288 -> 4096 9.6 + 9.6 -> 10.8 us) and the tables of a work-group's tiles do: the ones of the scale bytes, else 16-byte
+// ones, else (wider work-groups than the planned ones, by a tuning variable) the default codebook's 8-byte ones. What fits
+// none of them keeps the halves. Where the rows fit, LDS is faster: its work-groups share what every wave loads from L2
+// here (13 rows, gate/up 2 x 12288 x 4096: 14.8 against 17.0 us).
+int xg_table(const mdx_w4* const* ws, int nm, bool pair, int rows, bool other_src, bool tbl8) {
+    const mdx_w4& w = *ws[0];
+    if (rows <= 8 || int64_t(rows) * w.k <= 128 * 1024 || other_src || w.group_size < 16 || ilog2(w.group_size) < 0) return 0;
+    const bool bytes = w.s_dtype == MDX_DT_FP8E4M3 && w.group_size < 128;
+    if (!bytes && (w.decode == MDX_DECODE_INTEGRAL || w.group_size < 128 || w.k / w.group_size > 192)) return 0;
+    if (bytes && w.k / w.group_size > 2048) return 0;
+    GemvArgs a{};
+    int total = 0;
+    for (int i = 0; i < nm; ++i) {
+        if (!ws[i]) return 0;
+        total += int(ws[i]->n / 16);
+    }
+    a.K = int(w.k);
+    a.lgG = ilog2(w.group_size);
+    a.rows = rows;
+    a.xg = 1;
+    gemv_geometry(total, a.K, pair, 8, a.TPW, a.KS);
+    auto fits = [&](int tbl) {
+        a.tbl = tbl;
+        return gemv_smem(a, true, esz_of(w.s_dtype)) <= LDS_MAX;
+    };
+    if (bytes) return fits(3) ? 3 : 0;
+    if (!(tbl8 && !w.codebook) && fits(1)) return 1;
+    return !w.codebook && fits(2) ? 2 : 0;
 }
 
 // Extra activation sources and outputs of one launch (all optional).
@@ -1793,7 +1817,11 @@ int run_gemv(const mdx_w4* const* ws, int nm, bool pair, const int8_t* xq, const
     MDX_CHECK(!ex.gn_y || (nm == 1 && !pair && ex.gn_z && ex.gn_w && gemv_gn_fits(ws[0], rows)), "gated-norm GEMV geometry");
     // the table variants take many rows straight from L2 (SRC_XG); the others hold them in LDS: above 128 KiB, they run
     // the rows in two halves
-    const bool xg = xg_fits(*ws[0], rows, ex.hr || ex.xp_x || ex.gn_y || ex.gdn);
+    const TuneEnv tune;
+    const char* te = tune.get("MDX_GEMV_TBL");  // MDX_GEMV_TBL=8: the 8-byte tier whenever it applies (tests)
+    const bool tbl8_only = te && atoi(te) == 8;
+    const int xt = xg_table(ws, nm, pair, rows, ex.hr || ex.xp_x || ex.gn_y || ex.gdn, tbl8_only);
+    const bool xg = xt != 0;
     if (!xg && rows > 8 && int64_t(rows) * ws[0]->k > 128 * 1024) {
         const int ra = 8, rb = rows - 8;
         int rc = run_gemv(ws, nm, pair, xq, xs, ra, epi, outs, res, out_dt, lut, st);
@@ -1843,18 +1871,16 @@ int run_gemv(const mdx_w4* const* ws, int nm, bool pair, const int8_t* xq, const
         const int nw = a.TPW * a.KS;
         a.gf.nside = (rows * a.gf.HV + nw - 1) / nw;
     }
-    MDX_CHECK(xg || gemv_smem(a, mfma, esz) <= 160 * 1024, "activation of %d rows x K=%d exceeds LDS", rows, a.K);
+    MDX_CHECK(xg || gemv_smem(a, mfma, esz) <= LDS_MAX, "activation of %d rows x K=%d exceeds LDS", rows, a.K);
     // per-weight decode tables in LDS when the scales are not asserted integral, a group spans a chunk
     // and the larger footprint still holds the grid's work-groups per CU (else fewer resident: at 8
     // rows the gate/up pair would drop from three work-groups per CU to two and lose more than the
     // tables save; there the lanes build their tables in the loop). Tables select the table-only
     // variants, which run on the MFMA kernel at every row count (at one row too: the products leave
     // the VALU to the decode).
-    const TuneEnv tune;
-    const char* te = tune.get("MDX_GEMV_TBL");  // MDX_GEMV_TBL=8: the 8-byte tier whenever it applies (tests)
-    const bool tbl8 = te && atoi(te) == 8 && !a.cb;
-    if (xg && a.lgG >= 7) {
-        a.tbl = tbl8 ? 2 : 1;  // (without the rows in LDS a work-group's tables always leave room for others)
+    const bool tbl8 = tbl8_only && !a.cb;
+    if (xg) {
+        a.tbl = xt;
         mfma = true;
     } else if (!a.assume_int && a.lgG >= 7) {
         const int per_cu = (wgs + 255) / 256;
@@ -1865,10 +1891,10 @@ int run_gemv(const mdx_w4* const* ws, int nm, bool pair, const int8_t* xq, const
         for (int tb = tbl8 ? 2 : 1; tb <= 2; ++tb) {
             if (tb == 2 && a.cb) break;
             a.tbl = tb;
-            if (int64_t(per_cu) * gemv_smem(a, true, esz) <= 160 * 1024) break;
+            if (int64_t(per_cu) * gemv_smem(a, true, esz) <= LDS_MAX) break;
             if (tb == 1 && !ex.hr && !ex.xp_x && !ex.gn_y && size_t(a.TPW) * 16 * ngr * 16 >= red_bytes) {
                 a.red_alias = 1;
-                if (int64_t(per_cu) * gemv_smem(a, true, esz) <= 160 * 1024) break;
+                if (int64_t(per_cu) * gemv_smem(a, true, esz) <= LDS_MAX) break;
                 a.red_alias = 0;
             }
             a.tbl = 0;
@@ -1878,13 +1904,12 @@ int run_gemv(const mdx_w4* const* ws, int nm, bool pair, const int8_t* xq, const
     // fp8 scales in groups below a chunk: the tables of the scale bytes at every row count (one row too: the
     // products leave the VALU to the decode). Only one row whose scales are asserted integral keeps its integral
     // form, which needs no table.
-    if (ws[0]->s_dtype == MDX_DT_FP8E4M3 && a.lgG < 7 &&
+    if (!xg && ws[0]->s_dtype == MDX_DT_FP8E4M3 && a.lgG < 7 &&
         !(rows == 1 && a.assume_int && !a.cb && !a.force_exact && a.lgG >= 5)) {
         a.tbl = 3;
-        if (gemv_smem(a, true, esz) <= 160 * 1024) mfma = true;
+        if (gemv_smem(a, true, esz) <= LDS_MAX) mfma = true;
         else a.tbl = 0;
     }
-    MDX_CHECK(!xg || (a.tbl && gemv_smem(a, true, esz) <= 160 * 1024), "rows from L2: tables within LDS");
     MDX_CHECK(!(mfma && a.xp_x) || a.tbl, "row-prep GEMV geometry (one row takes the VALU kernel or the tables)");
     // per-wave one-shots: one int8 row, caller-asserted integral scales with the default codebook,
     // G128, 16-byte runs of scales per slice and per row (MDX_GEMV_PWO=0 turns them off)

@@ -39,3 +39,28 @@ def test_rows_past_lds_match_oracle(C, dev, form, N, K, G, M, tiled):
     assert len(tr) == 1 and tr[0]["rows"] == M and tr[0]["decode"] in ("table16", "bytes"), tr
     want = ref.w4a8_linear(x.numpy(), xs.numpy(), q.numpy(), sf, sc.numpy(), None if cb is None else cb.numpy(), G, bits(res))
     assert_bits_equal(bits(out), np.asarray(want), "rows past LDS")
+
+
+@pytest.mark.parametrize("custom,decode", [(False, ["table8"]), (True, None)])
+def test_wide_work_groups_fall_back(C, dev, monkeypatch, custom, decode):
+    """Six tiles per work-group (a tuning variable): the 16-byte tables of 13 rows x 12288 pass LDS. The default codebook
+    takes 8-byte ones, another codebook the two halves, and neither is refused."""
+    from mdx import _lib, layout
+    monkeypatch.setenv("MDX_GEMV_TPW", "6")
+    N, K, G, M = 192, 12288, 128, 13
+    g = torch.Generator().manual_seed(6)
+    q = torch.randint(-128, 128, (N, K // 2), generator=g, dtype=torch.int8)
+    s = (torch.rand(N, K // G, generator=g) * 30).half()
+    sc = torch.rand(N, generator=g) * 1e-3 + 1e-4
+    cb = torch.randn(16, generator=g) * 4 if custom else None
+    x = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8)
+    xs = torch.rand(M, generator=g) * 0.05 + 1e-3
+    w = layout.W4(layout.tile_major_codes(q).to(dev), s.to(dev), sc.to(dev), None if cb is None else cb.to(dev), _lib.LAYOUT_TILE)
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    _lib.gemv_trace()
+    C.stream_gemv(x.to(dev), xs.to(dev), [w], [out])
+    tr = _lib.gemv_trace()
+    assert [r["rows"] for r in tr] == ([8, 5] if custom else [13]), tr
+    assert decode is None or [r["decode"] for r in tr] == decode, tr
+    want = ref.w4a8_linear(x.numpy(), xs.numpy(), q.numpy(), s.float().numpy(), sc.numpy(), None if cb is None else cb.numpy(), G)
+    assert_bits_equal(bits(out), np.asarray(want), "six tiles")
