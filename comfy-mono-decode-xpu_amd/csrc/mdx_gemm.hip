@@ -82,10 +82,10 @@ __device__ __forceinline__ uint32_t lds_u32(const void* p) {
 // one direct-to-LDS load: 16 (4) bytes per lane from base + off (ptr) to LDS bytes dst + 16 (4) lane
 __device__ __forceinline__ void dma16(uint32_t dst, const uint8_t* base, uint32_t off) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base)
-                 : "memory");
+                 : "memory", "m0");
 }
 __device__ __forceinline__ void dma4(uint32_t dst, const uint8_t* ptr) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(dst), "v"(ptr) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(dst), "v"(ptr) : "memory", "m0");
 }
 
 __device__ __forceinline__ int gmat(const GemmArgs& a, int g, int& tile) {
