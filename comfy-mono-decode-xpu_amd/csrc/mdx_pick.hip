@@ -15,7 +15,8 @@
 //   1. candidates: the work-group's S best approximate scores (ties: the smaller index). An element's key is
 //      32 bits, the bf16 value order above its place in the segment (at most 8192 elements). theta = the
 //      S-th largest of the maxima of the 64 quads of threads; every element >= theta belongs to a quad whose
-//      maximum is >= theta (S of them), then counting ranks. (64-bit keys and counting over 256 thread
+//      maximum is >= theta (S of them), then counting ranks. Where those are more than S threads could hold, theta
+//      comes from the thread maxima: at most 32 S candidates. (64-bit keys and counting over 256 thread
 //      maxima: 5.2 us to theta and 1.8 us to collect, of 21 us.)
 //   2. the candidates' exact logits: int8 (the 32 candidate rows and the activation land in LDS by DMA
 //      in K blocks of 4 KiB, then v_dot4 and a wave sum per candidate; integer, so any order), bf16
@@ -202,6 +203,7 @@ __global__ __launch_bounds__(PK_T) void draft_pick_kernel(PickArgs a) {
         key[j] = t + PK_T * j < len ? sel_key(v[j], uint32_t(t + PK_T * j)) : 0u;
         m = max(m, key[j]);
     }
+    const uint32_t mt = m;  // this thread's maximum
     m = max(m, quad_x<0xB1>(m));
     m = max(m, quad_x<0x4E>(m));
     if ((t & 3) == 0) qmax[t >> 2] = m;
@@ -221,12 +223,27 @@ __global__ __launch_bounds__(PK_T) void draft_pick_kernel(PickArgs a) {
         if ((t & 3) == 0 && above == uint32_t(a.S - 1)) theta = m;
     }
     __syncthreads();
-    const uint32_t th = theta;
+    auto collect = [&]() {
+        const uint32_t th = theta;
 #pragma unroll
-    for (int j = 0; j < PK_E; ++j)
-        if (key[j] >= th) cand[atomicAdd(&ncand, 1)] = key[j];  // (S quads hold such elements: below 4 S PK_E)
-    __syncthreads();
-    const int nc = ncand;
+        for (int j = 0; j < PK_E; ++j)
+            if (key[j] >= th) cand[atomicAdd(&ncand, 1)] = key[j];  // (S quads hold such elements: below 4 S PK_E)
+        __syncthreads();
+        return ncand;
+    };
+    int nc = collect();
+    if (nc > a.S * PK_E) {
+        // (uniform) scores so regular that a few quads hold most of the best ones, up to 4 S PK_E of them, which the
+        // ranks below would count against each other: theta from the 256 thread maxima instead, S threads' elements at
+        // most (262144 scores, 64 of every 256 far above the rest: 548 -> 18 us)
+        __syncthreads();
+        cand[t] = mt;
+        if (t == 0) ncand = 0;
+        __syncthreads();
+        if (count_above(cand, PK_T, mt) == a.S - 1) theta = mt;
+        __syncthreads();
+        nc = collect();
+    }
     for (int i = t; i < nc; i += PK_T) {
         const int pos = count_above(cand, nc, cand[i]);
         if (pos < a.S) sel[pos] = int(s0) + int(0xFFFFu - (cand[i] & 0xFFFFu));

@@ -134,3 +134,26 @@ def test_draft_pick_bf16_odd_k(C, dev, tiled):
             assert torch.equal(vals.view(torch.int16), wv.view(-1).view(torch.int16)), (trial, nout)
             want_tok = C.fast_topk(logits, 1, True)[1].item() if amf else wi.view(-1)[0].item()
             assert token.item() == want_tok
+
+
+@pytest.mark.parametrize("N", [65536, 151936, 262144])
+@pytest.mark.parametrize("columns", [4, 60, 64, 128, 256])
+def test_draft_pick_of_regular_scores(C, dev, N, columns):
+    """Scores with a period of 256 (the width of the pick's sweep): the first `columns` of each period hold all the good
+    ones, so that a few threads hold most of a segment's best elements."""
+    g = torch.Generator().manual_seed(N + columns)
+    x = torch.randn(N, generator=g) - 20
+    seg = -(-N // 32)
+    i = torch.arange(N) % seg  # place within the work-group's segment
+    good = i % 256 < columns
+    x[good] = (torch.randn(int(good.sum()), generator=g) + 10).abs()
+    approx = x.bfloat16().to(dev)
+    e8, ef32 = torch.empty(0, dtype=torch.int8, device=dev), torch.empty(0, dtype=torch.float32, device=dev)
+    exact = bits(approx)
+    for nout in (1, 8):
+        print(f"case pick regular N={N} columns={columns} nout={nout}", flush=True)
+        top = torch.full((nout,), -1, dtype=torch.long, device=dev)
+        token, vtok = torch.full((1,), -1, dtype=torch.long, device=dev), torch.full((8,), -1, dtype=torch.long, device=dev)
+        C.draft_pick(approx, e8, ef32, e8, ef32, nout, False, top, top[:0], token, vtok, [1], None)
+        wtop, wtok, _ = ref.draft_pick(exact, nout, False, [1], 8)
+        assert top.tolist() == wtop.tolist() and token.item() == wtok
