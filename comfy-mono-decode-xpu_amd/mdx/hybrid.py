@@ -291,6 +291,7 @@ class HybridModel:
         # host-side upper bound of the committed position st[0]: every KV write of a step lands at
         # most R - 1 past it, and each step commits at most len(widths) + 1 tokens
         self.pos_bound = None
+        self.parity = 0  # of the next step: the rows pending before it lie in the other parity's buffers
         # a list to receive (name, copy) of the step's intermediates (eager steps only; None: off)
         self.trace = None
 
@@ -685,11 +686,13 @@ class HybridModel:
             raise RuntimeError(f"prompt of {prompt.numel()} tokens: needs 2 <= tokens and tokens + {self.R} tree rows "
                                f"<= the cache capacity {c.cap}")
         body = prompt[:-1]
-        n0, parity = 0, 0
+        # rows pending from an earlier prompt or decode step lie in the buffers of the other parity
+        n0, parity = 0, self.parity
         last = (body.numel() - 1) // S  # the last chain's number
         if last > 0 and self._run_fits():
-            total, parity = body.numel(), last & 1
-            self.ctl[1:2].zero_()  # (a first chain's parity: rows pending from a decode step are replayed from the other's buffers)
+            total = body.numel()
+            self.ctl[1:2].fill_(parity)
+            parity = (parity + last) & 1  # the last chain's
             while n0 < total:
                 n = total - n0 if total - n0 <= self.RUN_ROWS + S else self.RUN_ROWS  # (whole chains, the last with rows before it)
                 tail = total - last * S if n0 + n == total else 0

@@ -1,0 +1,121 @@
+"""The prompt prefill over several runs of rows (RUN_ROWS lowered so that short prompts take three and more), against the
+same prompt in chains of `slots`."""
+import pytest
+import torch
+
+from conftest import assert_bits_equal, bits
+
+pytestmark = pytest.mark.gpu
+
+RUN = 32
+
+
+def _pair(dev, monkeypatch, bodies, layers, **kw):
+    """The same prompts through the runs and through the chains; returns both models."""
+    from mdx import hybrid
+    ms = []
+    for run in (True, False):
+        cfg = hybrid.HybridConfig(layers=layers, inter=4096, vocab=32768, cap=512, greedy=True, **kw)
+        m = hybrid.HybridModel(cfg, dev, seed=9)
+        calls = []
+        f = m._prefill_run
+        m._prefill_run = lambda tokens, *a, _f=f, _c=calls: _c.append(tokens.numel()) or _f(tokens, *a)
+        g = torch.Generator().manual_seed(sum(bodies))
+        with monkeypatch.context() as mp:
+            mp.setattr(hybrid.HybridModel, "RUN_ROWS", RUN)
+            if run:
+                assert m._run_fits()
+            else:
+                mp.setattr(hybrid.HybridModel, "_run_fits", lambda self: False)
+            for n in bodies:
+                del calls[:]
+                m.prefill(torch.randint(0, cfg.vocab, (n + 1,), generator=g))
+                m.pos_bound = int(m.st[0].item())
+                if run:
+                    full = -(-max(n - RUN - cfg.slots, 0) // RUN)  # (runs of RUN rows while more than RUN + slots are left)
+                    assert calls == [RUN] * full + [n - RUN * full], calls
+                else:
+                    assert not calls
+        ms.append(m)
+    return ms
+
+
+def _same_state(a, b, what):
+    assert torch.equal(a.st, b.st) and torch.equal(a.ctl, b.ctl) and torch.equal(a.nt, b.nt) and a.parity == b.parity, what
+    assert_bits_equal(bits(a.hbuf), bits(b.hbuf), f"{what} hidden row")
+    p = a.parity ^ 1  # the last chain's buffers, which the first decode step replays
+    for i, (x, y) in enumerate(zip(a.gdn, b.gdn)):
+        for n in ("rec", "conv") if x is not None else ():
+            assert_bits_equal(bits(x[n]), bits(y[n]), f"{what} layer {i} {n}")
+        for n in ("pb", "qb", "gates") if x is not None else ():
+            assert_bits_equal(bits(x[n][p]), bits(y[n][p]), f"{what} layer {i} {n}")
+    n = int(a.st[1].item())
+    for x, y in zip(a.mkv, b.mkv):
+        assert_bits_equal(bits(x[:, :, :n]), bits(y[:, :, :n]), f"{what} draft block cache")
+
+
+# around the ends of a run: whole runs, one row more, a last run of RUN + slots rows and the first one past it
+@pytest.mark.parametrize("slots,kw", [(16, {}), (8, dict(widths=(3,)))])
+@pytest.mark.parametrize("k", [1, 3])
+@pytest.mark.parametrize("more", ["0", "1", "slots", "slots+1"])
+def test_runs_leave_the_chains_bits(dev, monkeypatch, slots, kw, k, more):
+    """Gated-DeltaNet layers only: the state after several runs is the chains' bit for bit."""
+    n = k * RUN + {"0": 0, "1": 1, "slots": slots, "slots+1": slots + 1}[more]
+    print(f"case runs slots={slots} rows={n}", flush=True)
+    a, b = _pair(dev, monkeypatch, [n], 3, slots=slots, **kw)
+    _same_state(a, b, f"{n} rows")
+
+
+@pytest.mark.parametrize("bodies", [[97, 70], [49, 113], [20, 96]])
+def test_runs_of_a_second_prompt(dev, monkeypatch, bodies):
+    """The second prompt's first run starts with rows pending from the first prompt, its others with none."""
+    a, b = _pair(dev, monkeypatch, bodies, 3)
+    _same_state(a, b, f"{bodies} rows")
+
+
+@pytest.mark.parametrize("run", [True, False])
+@pytest.mark.parametrize("first,second", [(10, 60), (20, 60), (40, 7), (97, 70)])
+def test_two_prompts_equal_one(dev, monkeypatch, run, first, second):
+    """A prompt fed in two pieces (the second starts with the first's last token) and the first decode step after it: the
+    rows that the first piece leaves pending are replayed from its buffers, whichever parity they have."""
+    from mdx import hybrid
+    cfg = hybrid.HybridConfig(layers=3, inter=4096, vocab=32768, cap=512, greedy=True)
+    if not run:
+        monkeypatch.setattr(hybrid.HybridModel, "_run_fits", lambda self: False)
+    tokens = torch.randint(0, cfg.vocab, (first + second + 1,), generator=torch.Generator().manual_seed(first))
+    ms = []
+    for pieces in ([tokens], [tokens[:first + 1], tokens[first:]]):
+        m = hybrid.HybridModel(cfg, dev, seed=9)
+        for t in pieces:
+            m.prefill(t)
+        m.pos_bound = first + second
+        ms.append(m)
+    a, b = ms
+    assert torch.equal(a.st, b.st) and torch.equal(a.nt, b.nt)
+    assert_bits_equal(bits(a.hbuf), bits(b.hbuf), "hidden row")
+    for m in ms:
+        m.step(m.parity)
+    assert_bits_equal(bits(a.logits), bits(b.logits), "logits")
+    assert torch.equal(a.result, b.result) and torch.equal(a.st, b.st)
+    for i, (x, y) in enumerate(zip(a.gdn, b.gdn)):
+        for n in ("rec", "conv"):
+            assert_bits_equal(bits(x[n]), bits(y[n]), f"layer {i} {n}")
+
+
+@pytest.mark.parametrize("n", [96, 97, 112, 113, 200])
+def test_runs_with_attention(dev, monkeypatch, n):
+    """With an attention layer the order of its fp32 sums differs from the chains', and a bf16 rounding that flips travels
+    through the layers that follow: states, caches and the first decode step's logits within TOL of the chains'."""
+    a, b = _pair(dev, monkeypatch, [n], 4)
+    assert torch.equal(a.st, b.st) and torch.equal(a.ctl, b.ctl) and torch.equal(a.nt, b.nt) and a.parity == b.parity
+    pairs = [(x[:, :, :n], y[:, :, :n]) for u, w in zip(a.kv + [a.mkv], b.kv + [b.mkv]) if u is not None for x, y in zip(u, w)]
+    pairs += [(x["rec"], y["rec"]) for x, y in zip(a.gdn, b.gdn) if x is not None] + [(a.hbuf, b.hbuf)]
+    rel = [float((x.double() - y.double()).norm() / y.double().norm()) for x, y in pairs]
+    for m in (a, b):
+        m.step(m.parity)
+    lg = float((a.logits.double() - b.logits.double())[0].norm() / b.logits.double()[0].norm())
+    print(f"case attention rows={n}: largest {max(rel):.2e}, logits {lg:.2e}", flush=True)
+    assert max(rel) <= TOL and lg <= TOL
+
+
+TOL = 2e-3
