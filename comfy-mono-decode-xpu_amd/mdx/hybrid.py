@@ -219,6 +219,19 @@ class HybridModel:
             cbs = [ws[r].cb for r in ("g", "u", "d")]
             if not (all(cb is None for cb in cbs) or all(cb is not None and torch.equal(cb, cbs[0]) for cb in cbs)):
                 raise ValueError(f"layer {i}: gate / up / down codebooks differ")
+            # one codebook buffer for the linears of a launch (libmdx compares its address), none for code - 8
+            for group in (("g", "u", "d"), ("q", "k", "v"), ("qkv", "z"), ("o",)):
+                shared = None
+                for r in group:
+                    w = ws.get(r)
+                    if w is None or w.cb is None:
+                        continue
+                    cb = _C._codebook(w.cb)
+                    if cb is not None and shared is not None and torch.equal(cb, shared):
+                        cb = shared
+                    shared = cb if shared is None else shared
+                    if cb is not w.cb:
+                        ws[r] = layout.W4(w.q, w.s, w.sc, cb, w.layout, w.decode)
             self.layers[i].update(ws)
 
     # ---- decode state --------------------------------------------------------------------------
