@@ -14,15 +14,14 @@
 //                 the online softmax state of a row lives in its lanes;
 //   O^T += V^T P^T   A = V^T, its 8 k-slots per lane in the token order the S^T accumulators hold,
 //                 B = bf16(P^T) straight from the S^T registers -- no shuffle of P.
-// Each work-group stores a chunk partial (m, l, O in fp32); attn_merge_kernel (one work-group per
-// query row, one thread per dim) combines the chunks and the tree-row partial and writes bf16. The
-// context split is recomputed on the device from seqlen in both launches, so a captured graph
-// replays for any context length.
+// Each work-group stores a chunk partial (m, l, O in fp32); attn_merge_kernel (one work-group of 256 per
+// query row) combines the chunks and the tree-row partial and writes bf16. The context split is recomputed
+// on the device from seqlen in both launches, so a captured graph replays for any context length.
 //
 // One work-group per (kv head, chunk) over all of the kv head's row tiles, K/V read once from HBM into an LDS ring (see
 // the layout note at stage_k). Head_dim 256 (4 kv heads, 8 rows of 4 heads, ctx 8192): 14.0 us per launch (13.7 without
-// the maximum per stage, add_own_max); with K rows
-// straight from HBM as MFMA operands, V transposed through LDS and a work-group per (row tile, chunk) it took 23.9 us.
+// the maximum per stage, add_own_max); with K rows straight from HBM as MFMA operands, V transposed through LDS and a
+// work-group per (row tile, chunk) it took 23.9 us.
 //
 // The tree-verify form with the Q/K prep (attn2_kernel<.., PREP>, head_dim 128): the launch also does the
 // RoPE/KV kernel's work for these rows (mdx_rope.hpp: per-head RMSNorm, split-half RoPE), so the step
@@ -839,8 +838,8 @@ int launch_prefill(const AttnArgs& a, hipStream_t st) {
 }
 
 int stream_rtw(int RT) { return RT <= 1 ? 1 : (RT == 2 ? 2 : 4); }
-// token parts per chunk (head_dim 256: a stage is 32 KiB, so two parts of two stages, or one of four with four row tiles):
-// eight waves per work-group (two per SIMD, so one wave's LDS and MFMA waits
+// token parts per chunk (head_dim 256: a stage is 32 KiB, so two parts of two stages, or one of four with four row tiles;
+// two waves with one row tile, else four): eight waves per work-group (two per SIMD, so one wave's LDS and MFMA waits
 // overlap the other's work) where each part still gets two ring stages, else four waves (head_dim 128
 // with one row tile)
 int stream_parts(int D, int RT) {

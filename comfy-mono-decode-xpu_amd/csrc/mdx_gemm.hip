@@ -11,9 +11,10 @@
 // the MFMAs of a stage freely (with the builtin it waits for every direct-to-LDS load in flight before any LDS
 // read, which drains the ring at each stage). The kernel waits itself: s_waitcnt vmcnt, then s_barrier, per stage.
 //
-// Bound by the decode's VALU work beside the products (about 75 instructions per 16 x 128 codes against 32 MFMAs of a
-// wave's stage). 1000 rows, K = 4096: gate/up 2 x 12288 columns 142 us (1.42 POP/s), 12288 columns 89 us; 4096 columns
-// with two waves per SIMD (KSP) 32 us against 41 us with one. The same 1000 rows through the decode kernels: 63 x 16 rows,
+// Bound by a stage's parts one after another (operand reads, the decode of about 75 VALU per 16 x 128 codes, 32 MFMAs of
+// a wave) behind one barrier: no single part taken out gains more than a fifth (gate/up 140 us; without the decode 127,
+// without 7/8 of the MFMAs 115, without operand reads 140, without loads 132). 1000 rows, K = 4096: gate/up 2 x 12288
+// columns 140 us (1.44 POP/s), 12288 columns 87 us; 4096 columns with two waves per SIMD (KSP) 32 us against 41 us with one. The same 1000 rows through the decode kernels: 63 x 16 rows,
 // 1.0 ms for the gate/up pair.
 //
 // Products: v_mfma_i32_16x16x64_i8 (exact int32 sums: the bits are the GEMV's) or v_mfma_f32_16x16x32_bf16, A = 16

@@ -144,7 +144,8 @@ __global__ __launch_bounds__(256) void gdn_run_prep_kernel(RunArgs a) {
 // The delta rule over the run: work-group (value head h, 16 state columns), thread (row group rg, column) as in
 // gdn_head_kernel. The rows come in blocks of 16: thread t holds piece t % 16 (8 elements) of row t / 16's k and q, so
 // the norms and k . q are sums over 16 lanes (halving trees) and the scaled rows go to LDS, double-buffered: the block
-// after next is in flight from memory while the waves walk one. Bound by the serial walk, about 0.2 us a row.
+// after next is in flight from memory while the waves walk one. Bound by the serial walk, 0.27 us a row
+// (1000 rows 274 us).
 constexpr int SC = 16, RG = 8, EB = 16;
 
 __device__ __forceinline__ float ror4_sum(float v) {

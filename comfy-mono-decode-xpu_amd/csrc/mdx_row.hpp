@@ -37,8 +37,8 @@ __device__ __forceinline__ double h4_out(const double* a, int j) {
     return __dadd_rn(__dadd_rn(__dadd_rn(b[0], b[1]), b[2]), b[3]);
 }
 
-// v of this lane in the banks (quads of each row of 16) of BANKS, w of the lane that DPP control CTRL names in the
-// others' place: one v_mov_b32_dpp per 32-bit half
+// w of the lane that DPP control CTRL names in the banks (quads of each row of 16) of BANKS, v of this lane in the
+// others: one v_mov_b32_dpp
 template <int CTRL, int BANKS>
 __device__ __forceinline__ uint32_t dpp_banks(uint32_t v, uint32_t w) {
     return uint32_t(__builtin_amdgcn_update_dpp(int(v), int(w), CTRL, 0xF, BANKS, false));

@@ -264,9 +264,8 @@ size_t mdx_attn_workspace(int64_t H, int64_t Hk, int64_t S, int64_t D, int64_t c
  * contiguous; xk/xv bf16 [Hk, S, D] (head / row strides as given, each); mask int32 [S]; out bf16
  * [S, H, D].
  * D in {64, 128, 256}; 1 <= S <= 16; (H / Hk) * S <= 64. seqlen is read on the device.
- * chunks_hint: 0 plans the context split (chunks of >= 128 tokens per wave); n > 0 splits the context
- * into at most n chunks per kv head of >= 32 tokens per wave (as the reference's chunks_hint steers
- * its split). */
+ * chunks_hint: 0 plans the context split (one round of work-groups, chunks of whole 32-token stages); n > 0
+ * caps it at n chunks per kv head (as the reference's chunks_hint steers its split). */
 int mdx_attn_decode(const uint16_t* q, int64_t q_head_stride, int64_t q_row_stride, const uint16_t* key,
                     const uint16_t* value, const int32_t* seqlen, const uint16_t* xk, int64_t xk_head_stride,
                     int64_t xk_row_stride, const uint16_t* xv, int64_t xv_head_stride, int64_t xv_row_stride,
