@@ -695,9 +695,10 @@ class HybridModel:
         S = c.slots
         dev = self.dev
         prompt = prompt.to(dev)
-        if prompt.numel() < 2 or prompt.numel() + self.R > c.cap:
-            raise RuntimeError(f"prompt of {prompt.numel()} tokens: needs 2 <= tokens and tokens + {self.R} tree rows "
-                               f"<= the cache capacity {c.cap}")
+        st0 = int(self.st[0].item())  # positions taken by what came before in the sequence
+        if prompt.numel() < 2 or st0 + prompt.numel() + self.R > c.cap:
+            raise RuntimeError(f"prompt of {prompt.numel()} tokens at position {st0}: needs 2 <= tokens and position + "
+                               f"tokens + {self.R} tree rows <= the cache capacity {c.cap}")
         body = prompt[:-1]
         # rows pending from an earlier prompt or decode step lie in the buffers of the other parity
         n0, parity = 0, self.parity
@@ -738,9 +739,9 @@ class HybridModel:
             parity ^= 1
             self.hbuf.copy_(x[n - 1:n])
             n0 += n
-        self.nt.fill_(int(prompt[-1].item()))
+        self.nt.copy_(prompt[-1:].view(1, 1))
         self.parity = parity
-        self.pos_bound = body.numel()
+        self.pos_bound = st0 + body.numel()
 
     # ---- graphs ----------------------------------------------------------------------------------
     def _warm(self):

@@ -54,7 +54,6 @@ def _pair(dev, monkeypatch, bodies, layers, fp8=None, **kw):
             for n in bodies:
                 del calls[:]
                 m.prefill(torch.randint(0, cfg.vocab, (n + 1,), generator=g))
-                m.pos_bound = int(m.st[0].item())
                 if run:
                     full = -(-max(n - RUN - cfg.slots, 0) // RUN)  # (runs of RUN rows while more than RUN + slots are left)
                     assert calls == [RUN] * full + [n - RUN * full], calls
@@ -112,7 +111,6 @@ def test_two_prompts_equal_one(dev, monkeypatch, run, first, second):
         m = hybrid.HybridModel(cfg, dev, seed=9)
         for t in pieces:
             m.prefill(t)
-        m.pos_bound = first + second
         ms.append(m)
     a, b = ms
     assert torch.equal(a.st, b.st) and torch.equal(a.nt, b.nt)
@@ -124,6 +122,27 @@ def test_two_prompts_equal_one(dev, monkeypatch, run, first, second):
     for i, (x, y) in enumerate(zip(a.gdn, b.gdn)):
         for n in ("rec", "conv"):
             assert_bits_equal(bits(x[n]), bits(y[n]), f"layer {i} {n}")
+
+
+@pytest.mark.parametrize("run", [True, False])
+def test_a_second_prompt_counts_the_first(dev, monkeypatch, run):
+    """The capacity that a prompt needs starts at the position before it, and so does the bound that decode steps are held
+    to: past the cache neither a prompt nor a step is launched."""
+    from mdx import hybrid
+    if not run:
+        monkeypatch.setattr(hybrid.HybridModel, "_run_fits", lambda self: False)
+    cfg = hybrid.HybridConfig(layers=1, inter=4096, vocab=32768, cap=128, greedy=True)
+    m = hybrid.HybridModel(cfg, dev, seed=9)
+    tokens = torch.randint(0, cfg.vocab, (cfg.cap,), generator=torch.Generator().manual_seed(1))
+    m.prefill(tokens[:70])
+    st = m.st.clone()
+    with pytest.raises(RuntimeError, match="position 69"):
+        m.prefill(tokens[:cfg.cap - 69 - m.R + 1])
+    assert torch.equal(m.st, st)
+    m.prefill(tokens[:cfg.cap - 69 - m.R])
+    assert m.pos_bound == int(m.st[0].item()) == cfg.cap - m.R - 1
+    with pytest.raises(RuntimeError, match="cache capacity"):
+        m.step(m.parity)
 
 
 @pytest.mark.parametrize("codebook,n", [("own", 20), ("own", 113), ("default", 113)])
